@@ -1,0 +1,77 @@
+"""The FP64 loops that interpolate the fitted kernel table (long lists) against the loops
+that read the table itself, one lane per target in list order (SPHX_OPT_LOOP_SHAPE_FP64 = 1),
+on the same particles.
+
+Tolerances, fixed by rounding: a sum of 800 positive terms regrouped, over weights that agree
+to 2^-48, differs by at most 800 * 2^-52 + 2^-48 = 2e-13 relative (rho, xm, kx: 1e-12); the
+other fields are differences of such sums, bounded at 1e-10 of their largest magnitude as in
+the other FP64 tests.
+"""
+import numpy as np
+import pytest
+import torch
+
+from tests.helpers import uniform_box
+
+pytestmark = pytest.mark.gpu
+
+POSITIVE = ("rho", "xm", "kx")
+GROUPS = (("ax", "ay", "az"), ("c11", "c22", "c33", "c12", "c13", "c23"))
+STD = ("rho", "c11", "c12", "c13", "c22", "c23", "c33", "ax", "ay", "az", "du")
+VE = ("xm", "kx", "gradh", "c11", "c12", "c13", "c22", "c23", "c33", "divv", "curlv", "alpha", "ax", "ay", "az", "du")
+
+
+def field(step, f):
+    owner = step.ve if hasattr(step, "ve") and hasattr(step.ve, f) and getattr(step.ve, f) is not None else step.d
+    return getattr(owner, f).double().clone()
+
+
+# smooth: the kernel's own tables, every segment fitted.  rough: entries perturbed by 1e-3,
+# no segment reproduced by the fit.  patch: one perturbed entry in the first, a middle and
+# the last (shortened) segment.
+@pytest.mark.parametrize("table", ["smooth", "rough", "patch"])
+@pytest.mark.parametrize("kind", ["std", "ve"])
+@pytest.mark.parametrize("periodic", [True, False])
+def test_fitted_table_loops_equal_table_loops(kind, table, periodic):
+    from sphexa_amd import hydro
+    from sphexa_amd._lib import FP64
+
+    print("case", kind, table, periodic, flush=True)
+    inp, b = uniform_box(330_007, seed=11, periodic=periodic, ng=800)
+    box = hydro.make_box([b.xmin, b.ymin, b.zmin], [b.xmax, b.ymax, b.zmax], [b.bx, b.by, b.bz])
+    fields = STD if kind == "std" else VE
+    out = []
+    for shape in (0, 1):
+        ctx = hydro.Context(0)
+        try:
+            ctx.set_loop_shape(FP64, shape)
+            make = hydro.HydroStep if kind == "std" else hydro.VeHydroStep
+            step = make(ctx, len(inp["x"]), box, FP64, ng0=800, ngmax=1200)
+            tables = [step.d.wh] + ([step.ve.whd] if kind == "ve" else [])
+            for k, t in enumerate(tables):
+                n = t.numel()
+                noise = torch.from_numpy(np.random.default_rng(k).uniform(-1e-3, 1e-3, n)).to(t.device)
+                if table == "rough":
+                    t.add_(noise * t.abs().max())
+                elif table == "patch":
+                    for e in (3, n // 2, n - 2):
+                        t[e] += noise[e] * t.abs().max()
+            d_inp = {k: torch.from_numpy(np.ascontiguousarray(v)).to("cuda") for k, v in inp.items()}
+            if kind == "ve":
+                d_inp["alpha"] = torch.full_like(d_inp["x"], 0.3)
+            step.compute_forces(d_inp)
+            assert ctx.candidate_tests() >= 3e8  # the lists are long enough for the fitted form
+            out.append({f: field(step, f) for f in fields})
+            out[-1]["dt"] = step.d.minDtCourant
+        finally:
+            ctx.close()
+    got, ref = out
+    for f in fields:
+        assert torch.isfinite(ref[f]).all(), f
+        err = (got[f] - ref[f]).abs()
+        if f in POSITIVE:
+            assert (err / ref[f].abs()).max().item() < 1e-12, f
+        else:
+            group = next((g for g in GROUPS if f in g), (f,))
+            assert err.max().item() < 1e-10 * max(ref[g].abs().max().item() for g in group), f
+    assert abs(got["dt"] - ref["dt"]) < 1e-12 * ref["dt"]
