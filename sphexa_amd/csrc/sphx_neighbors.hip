@@ -42,7 +42,8 @@ struct NsFlags
     uint32_t           badGroup;   // a group with more than 64 particles
     uint32_t           retryCount; // groups that exceeded the small traversal capacities
     uint32_t           hfacMiss;   // a count to update h from lies beyond the factor table
-    unsigned long long tests;      // exact (target, candidate) distance tests of this pass
+    unsigned long long tests;      // (target, candidate) distance tests of this pass
+    uint32_t           overCount;  // groups that nsCandidates leaves to nsCandidatesExact
 };
 
 __device__ inline bool nodeOverlapsBox(const double* __restrict__ centers, const double* __restrict__ sizes, int node,
@@ -59,6 +60,50 @@ __device__ inline bool nodeOverlapsBox(const double* __restrict__ centers, const
     return ov;
 }
 
+// What nsCandidates needs of a group's search box
+struct GroupSearch
+{
+    double   cx, cy, cz, inv;  // its centre, and the scale of the FP32 coordinates: 1 over its largest half-width
+    float    hwx, hwy, hwz;    // half-widths of the targets' bounding box, scaled and widened
+    float    lim;              // a candidate farther than sqrt(lim) from that box has no hits
+    float    undecided;        // width of the shell in which FP32 results are not trusted
+    uint32_t fold, exact;      // candidates take the image nearest the centre; left to nsCandidatesExact
+    uint32_t pad;
+};
+__device__ inline GroupSearch groupSearch(const double gc[3], const double gh[3], double rmin, double rmax, const DBox& box,
+                                          bool exact)
+{
+    // candidates are folded to the image nearest the centre where the box leaves a periodic
+    // domain; a box over half the domain's length has no single nearest image
+    GroupSearch  b{};
+    const double S    = fmax(fmax(gh[0], gh[1]), gh[2]);
+    bool         fold = false;
+    exact             = exact || !(S > 0x1p-100 && S < 0x1p100);
+    for (int d = 0; d < 3; ++d)
+    {
+        if (!box.pbc[d]) continue;
+        fold  = fold || gc[d] - gh[d] < box.lo[d] || gc[d] + gh[d] > box.hi[d];
+        exact = exact || gh[d] >= 0.4999 * box.len[d];
+    }
+    b.cx = gc[0], b.cy = gc[1], b.cz = gc[2], b.inv = 1.0 / S;
+    // 2^-20 covers the rounding of the half-widths, 2^-17 that of the distances
+    b.hwx = fmaxf(float((gh[0] - rmin) * b.inv), 0.f) + 0x1p-20f;
+    b.hwy = fmaxf(float((gh[1] - rmin) * b.inv), 0.f) + 0x1p-20f;
+    b.hwz = fmaxf(float((gh[2] - rmin) * b.inv), 0.f) + 0x1p-20f;
+    const float rf = float(rmax * b.inv);
+    b.lim          = rf * rf + 0x1p-17f;
+    // Half-width of the shell around d^2 = (2h)^2 in which the FP32 result is not trusted.  With
+    // Q = max |e|^2 and T = max |t|^2 over the box: three roundings (2^-24 each) of a coordinate
+    // move d^2 by at most 2^-24 * 18 (Q + T) near the sphere; |e|^2, |t|^2 and (2h)^2 are off by
+    // 2^-24 of 3 Q, 3 T and 1; the products and sums, none over 2 (Q + T), by 8 roundings in any
+    // order: together below 2^-24 * (37 (Q + T) + 1).  Half as much again is used.
+    const float ux = b.hwx + rf, uy = b.hwy + rf, uz = b.hwz + rf;
+    const float QT = ux * ux + uy * uy + uz * uz + b.hwx * b.hwx + b.hwy * b.hwy + b.hwz * b.hwz;
+    b.undecided    = 2.f * (0x1p-24f * (56.f * QT + 2.f));
+    b.fold = fold, b.exact = exact;
+    return b;
+}
+
 // The ranges of one group g (all 64 lanes of the wave call this).  A group whose walk
 // exceeds the capacities gets no ranges and is appended to retryList, or, without a
 // retry list, raises the overflow flag.
@@ -68,8 +113,8 @@ __device__ void groupRangesOf(uint32_t g, GroupsDev G, const double* __restrict_
                               const int32_t* __restrict__ childOffsets, const int32_t* __restrict__ internalToLeaf,
                               const uint32_t* __restrict__ layout, const double* __restrict__ centers,
                               const double* __restrict__ sizes, const DBox& box, uint2* __restrict__ ranges,
-                              uint32_t* __restrict__ rangeCount, uint32_t* __restrict__ retryList,
-                              NsFlags* __restrict__ flags)
+                              uint32_t* __restrict__ rangeCount, GroupSearch* __restrict__ search,
+                              uint32_t* __restrict__ retryList, NsFlags* __restrict__ flags)
 {
     static_assert((LCAP & (LCAP - 1)) == 0 && LCAP <= NS_LCAP, "leaf capacity: a power of two within the range stride");
     __shared__ int32_t front[2][FCAP];
@@ -86,7 +131,7 @@ __device__ void groupRangesOf(uint32_t g, GroupsDev G, const double* __restrict_
     uint32_t i   = s + lane;
     bool     act = i < e;
 
-    double lo[3], hi[3];
+    double lo[3], hi[3], rmin, rmax;
     {
         double px[3] = {0, 0, 0};
         double r     = 0;
@@ -101,6 +146,8 @@ __device__ void groupRangesOf(uint32_t g, GroupsDev G, const double* __restrict_
             lo[d] = waveMin(act ? px[d] - r : INFINITY);
             hi[d] = waveMax(act ? px[d] + r : -INFINITY);
         }
+        rmin = waveMin(act ? r : INFINITY);
+        rmax = waveMax(act ? r : -INFINITY);
     }
     if (!(lo[0] <= hi[0]))
     {
@@ -209,28 +256,47 @@ __device__ void groupRangesOf(uint32_t g, GroupsDev G, const double* __restrict_
         }
     }
 
-    // ---- merge consecutive leaves into particle ranges
-    int rcount = 0;
-    for (int b = 0; b < lcount; b += 64)
-    {
-        int      k       = b + int(lane);
-        bool     inRange = k < lcount;
-        bool     isStart = inRange && (k == 0 || leafList[k] != leafList[k - 1] + 1);
-        uint64_t mS      = ballot(isStart);
-        int      r       = rcount + int(popc64(mS & lt));
-        if (isStart)
+    // ---- merge consecutive leaves into particle ranges, in pieces of at most 64 particles (the
+    // chunks of nsCandidates); more pieces than there is room for stay whole ranges
+    auto writeRanges = [&](uint32_t piece) {
+        int rcount = 0;
+        for (int b = 0; b < lcount; b += 64)
         {
-            // find the end of this run
-            int kk = k;
-            while (kk + 1 < lcount && leafList[kk + 1] == leafList[kk] + 1)
-                ++kk;
-            uint32_t ps = layout[leafList[k]];
-            uint32_t pe = layout[leafList[kk] + 1];
-            ranges[size_t(g) * NS_LCAP + r] = make_uint2(ps, pe);
+            const int  k       = b + int(lane);
+            const bool inRange = k < lcount;
+            const bool isStart = inRange && (k == 0 || leafList[k] != leafList[k - 1] + 1);
+            uint32_t   ps = 0, pe = 0;
+            if (isStart)
+            {
+                // find the end of this run
+                int kk = k;
+                while (kk + 1 < lcount && leafList[kk + 1] == leafList[kk] + 1)
+                    ++kk;
+                ps = layout[leafList[k]];
+                pe = layout[leafList[kk] + 1];
+            }
+            const int np  = pe > ps ? int((pe - ps - 1u) / piece + 1u) : 0;
+            int       sum = np;
+            for (int o = 1; o < 64; o <<= 1)
+            {
+                const int v = __shfl_up(sum, o, 64);
+                if (int(lane) >= o) sum += v;
+            }
+            int r = rcount + sum - np;
+            for (uint32_t c = ps; c < pe; ++r, c = pe - c > piece ? c + piece : pe)
+                if (r < NS_LCAP) ranges[size_t(g) * NS_LCAP + r] = make_uint2(c, pe - c > piece ? c + piece : pe);
+            rcount += __shfl(sum, 63, 64);
         }
-        rcount += int(popc64(mS));
+        return rcount;
+    };
+    int  rcount = writeRanges(64u);
+    bool exact  = rcount > NS_LCAP;
+    if (exact) rcount = writeRanges(~0u);
+    if (lane == 0)
+    {
+        rangeCount[g] = uint32_t(rcount);
+        search[g]     = groupSearch(gc, gh, rmin, rmax, box, exact);
     }
-    if (lane == 0) rangeCount[g] = uint32_t(rcount);
 }
 
 // all groups (or those of groupList) with the small capacities
@@ -244,12 +310,13 @@ __global__ __launch_bounds__(64) void nsGroupRanges(GroupsDev G, const uint32_t*
                                                     const double* __restrict__ centers,
                                                     const double* __restrict__ sizes, DBox box,
                                                     uint2* __restrict__ ranges, uint32_t* __restrict__ rangeCount,
+                                                    GroupSearch* __restrict__ search,
                                                     uint32_t* __restrict__ retryList, NsFlags* __restrict__ flags)
 {
     const uint32_t blk = xcdContiguous(blockIdx.x, gridDim.x);
     const uint32_t g   = groupList ? groupList[blk] : blk;
     groupRangesOf<Th, NS_FCAP_SMALL, NS_LCAP_SMALL>(g, G, x, y, z, h, childOffsets, internalToLeaf, layout, centers,
-                                                    sizes, box, ranges, rangeCount, retryList, flags);
+                                                    sizes, box, ranges, rangeCount, search, retryList, flags);
 }
 
 // the groups of the retry list with the large capacities (grid-stride over the list,
@@ -264,6 +331,7 @@ __global__ __launch_bounds__(64) void nsGroupRangesRetry(GroupsDev G, const doub
                                                          const double* __restrict__ centers,
                                                          const double* __restrict__ sizes, DBox box,
                                                          uint2* __restrict__ ranges, uint32_t* __restrict__ rangeCount,
+                                                         GroupSearch* __restrict__ search,
                                                          const uint32_t* __restrict__ retryList,
                                                          NsFlags* __restrict__ flags)
 {
@@ -271,12 +339,13 @@ __global__ __launch_bounds__(64) void nsGroupRangesRetry(GroupsDev G, const doub
     for (uint32_t k = blockIdx.x; k < n; k += gridDim.x)
     {
         groupRangesOf<Th, NS_FCAP, NS_LCAP>(retryList[k], G, x, y, z, h, childOffsets, internalToLeaf, layout,
-                                             centers, sizes, box, ranges, rangeCount, nullptr, flags);
+                                             centers, sizes, box, ranges, rangeCount, search, nullptr, flags);
         __syncthreads(); // the next group reuses the LDS lists
     }
 }
 
-// Candidate test.  Sph = true: findNeighborsSph semantics (nc counts self, h updates,
+// Candidate test with the predicate in FP64 for all pairs, of the groups that nsCandidates
+// leaves to it.  Sph = true: findNeighborsSph semantics (nc counts self, h updates,
 // redo flags) and the SPH list format below; Sph = false: findNeighbors semantics
 // (count without self, u32 lists in the reference CPU layout).
 //
@@ -302,7 +371,7 @@ constexpr uint32_t NS_QCAP = 128; // per-quarter queue capacity (ring buffer)
 __device__ int writeLane(int v, int lane, int old) __asm("llvm.amdgcn.writelane.i32");
 
 template<class Th, bool Sph>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6))) void nsCandidates(GroupsDev G, const uint32_t* __restrict__ groupList,
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6))) void nsCandidatesExact(GroupsDev G, const uint32_t* __restrict__ groupList,
                                                    const double* __restrict__ x, const double* __restrict__ y,
                                                    const double* __restrict__ z, Th* __restrict__ h,
                                                    uint8_t* __restrict__ iter, const uint2* __restrict__ ranges,
@@ -631,6 +700,443 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6))) void ns
     }
 }
 
+// The neighbor search proper.  One workgroup of 4 waves per target group, wave q for the 16
+// targets of quarter q.
+//
+//   filter : the group's candidate ranges are streamed in chunks of 64 particles, lane =
+//            candidate, 8 chunks at a time (two per wave).  A candidate within the group's
+//            largest 2h of the targets' bounding box is put, in ascending j, into an LDS ring:
+//            its position relative to the group's centre, in units of the search box's
+//            half-width, in FP32, and |e|^2.
+//   union  : every wave tests the ring's entries, 64 at a time, against its 16 targets with four
+//            MFMA (16x16x4 FP32): rows = targets (-2x, -2y, -2z, 1), columns = entries
+//            (x, y, z, |e|^2), C = |t|^2 - (2h)^2, so that the result is d^2 - (2h)^2.  Its
+//            minimum over the targets says whether the entry joins the quarter's union; the
+//            members are appended to a queue of the wave.
+//   masks  : 64 members of the queue at a time go through the MFMA again, rows = entries, columns =
+//            targets: a lane receives the results of 16 consecutive members for one target, whose
+//            sign bits are 16 bits of that target's mask, stored as they are.
+//
+// FP32 error bounds leave a shell around the sphere (about one pair in 30,000) where the
+// reference predicate d^2 < (2h)^2 is evaluated in FP64 with separately rounded operations
+// (findneighbors.hpp:33-60,115-140), so the neighbor sets are bit-identical to the CPU path.
+//
+// Groups without a single nearest periodic image, without a usable search box, or with a
+// target beyond ngmax neighbors (whose lists keep the first ngmax) are left to
+// nsCandidatesExact by overList.
+//
+// One wave per group with the predicate in FP64 for all pairs (nsCandidatesExact) took 4.66 ms at
+// 256^3 and 0.185 ms for 4,096 particles, where it leaves most of the chip idle; this takes 3.50
+// and 0.025 ms.  Bound by instruction issue: 1,250 VALU and 700 SALU instructions per wave, 60 %
+// of the time with VALU work, the rest waits for the first chunks and the barriers of a step.
+// candidate chunks per wave and step: 2 (1: 3.6 ms at 256^3, more steps; 3: 4.1, registers)
+constexpr uint32_t NS_PER_WAVE = 2;
+constexpr uint32_t NS_CHUNKS   = 4 * NS_PER_WAVE;     // per step
+constexpr uint32_t NS_RING     = 64 + 64 * NS_CHUNKS; // 63 entries carried over + a step's, whole batches
+// a wave's queue: two batches of 64 members (float4), 64 bytes of padding after each 16 of them
+// so that the masks' operand reads (members 16 apart) meet different banks
+constexpr uint32_t NS_QHALF = 64 * 4 + 4 * 16; // floats per batch
+
+using floatx4 = __attribute__((ext_vector_type(4))) float;
+
+// LDS written by other lanes of the same wave (whose LDS operations execute in order)
+__device__ inline void waveFence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// min(a, b) after exchanging the upper half of every 2 * Rows lanes of a with the lower half of
+// b's: the lower half then holds a's minima over both halves, the upper half b's
+template<int Rows>
+__device__ inline int swapMin(int a, int b)
+{
+    if constexpr (Rows == 32)
+    {
+        const auto v = __builtin_amdgcn_permlane32_swap(uint32_t(a), uint32_t(b), false, false);
+        return min(int(v[0]), int(v[1]));
+    }
+    else
+    {
+        const auto v = __builtin_amdgcn_permlane16_swap(uint32_t(a), uint32_t(b), false, false);
+        return min(int(v[0]), int(v[1]));
+    }
+}
+
+template<class Th, bool Sph>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void nsCandidates(
+    GroupsDev G, const uint32_t* __restrict__ groupList, const double* __restrict__ x, const double* __restrict__ y,
+    const double* __restrict__ z, Th* __restrict__ h, uint8_t* __restrict__ iter, const uint2* __restrict__ ranges,
+    const uint32_t* __restrict__ rangeCount, const GroupSearch* __restrict__ search, DBox box, uint32_t ngmax,
+    uint32_t ng0, HFactors hfac, uint32_t* __restrict__ nbrs, SphLists out, uint32_t* __restrict__ nc, uint32_t* __restrict__ redoList,
+    uint32_t* __restrict__ overList, NsFlags* __restrict__ flags, unsigned long long* __restrict__ groupTests)
+{
+#pragma clang fp contract(off)
+    __shared__ float4   ent[NS_RING];
+    __shared__ uint32_t entJ[NS_RING];
+    __shared__ float    queAll[4][2 * NS_QHALF];
+    __shared__ uint32_t queJAll[4][128];
+    __shared__ uint32_t selfAll[4][16]; // the union index of each target
+    __shared__ uint32_t wcnt[4], wflag[4];
+
+    const uint32_t blk  = xcdContiguous(blockIdx.x, gridDim.x);
+    const uint32_t g    = groupList ? groupList[blk] : blk;
+    const uint32_t q    = uint32_t(__builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6)));
+    const unsigned lane = threadIdx.x & 63u, part = lane >> 4, n = lane & 15u;
+    float*         que  = queAll[q];
+    uint32_t*      queJ = queJAll[q];
+    uint32_t       s, e;
+    groupRange(G, g, s, e);
+    if (e - s > 64) e = s + 64;
+    const uint32_t R = rangeCount[g];
+
+    if (R == 0 || search[g].exact)
+    {
+        if (threadIdx.x == 0)
+        {
+            overList[atomicAdd(&flags->overCount, 1u)] = g;
+            groupTests[blk]                            = 0;
+        }
+        return;
+    }
+    const GroupSearch sb   = search[g];
+    const float       invF = float(sb.inv);
+
+    // the wave's targets: lane 16 p + n holds target n (four copies)
+    const uint32_t i   = s + 16u * q + n;
+    const bool     act = i < e;
+    const double   px  = box.pbc[0] ? box.len[0] : 0.0;
+    const double   py  = box.pbc[1] ? box.len[1] : 0.0;
+    const double   pz  = box.pbc[2] ? box.len[2] : 0.0;
+    // the reference predicate for target ii; its fields are loaded anew (the empty asm keeps the
+    // loads and what follows from them here, off the common path's registers)
+    auto exactHit = [&](uint32_t ii, uint32_t j) {
+        asm volatile("" : "+v"(ii));
+        const double p[3] = {x[ii], y[ii], z[ii]}, hi = double(h[ii]);
+        double       dx = x[j] - p[0], dy = y[j] - p[1], dz = z[j] - p[2];
+        bool         inside = true;
+#pragma unroll
+        for (int d = 0; d < 3; ++d)
+            inside = inside && (p[d] - 2.0 * hi >= box.lo[d]) && (p[d] + 2.0 * hi <= box.hi[d]);
+        if (box.anyPbc && !inside)
+        {
+            dx -= px * rint(dx * box.ilen[0]);
+            dy -= py * rint(dy * box.ilen[1]);
+            dz -= pz * rint(dz * box.ilen[2]);
+        }
+        return dx * dx + dy * dy + dz * dz < 4.0 * hi * hi;
+    };
+
+    // MFMA operand of the targets and C; a target without neighbors (none, or not finite)
+    // gets +1e30 for every distance
+    float tx = 4.f, ty = 4.f, tz = 4.f, r2 = 0.f;
+    if (act)
+    {
+        const double rs = 2.0 * double(h[i]) * sb.inv;
+        tx = float(x[i] - sb.cx) * invF, ty = float(y[i] - sb.cy) * invF, tz = float(z[i] - sb.cz) * invF;
+        r2 = float(rs * rs);
+    }
+    const float undecided = sb.undecided;
+    const bool  usable = fabsf(tx) <= 2.f && fabsf(ty) <= 2.f && fabsf(tz) <= 2.f;
+    const float tval   = part == 3 ? 1.f : !usable ? 0.f : -2.f * (part == 0 ? tx : part == 1 ? ty : tz);
+    const float c0     = usable ? tx * tx + ty * ty + tz * tz - r2 + 0.5f * undecided : 1e30f;
+    const floatx4 cCol = {c0, c0, c0, c0};
+    floatx4       cRow; // of targets 4 part + k
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+        cRow[k] = __shfl(c0, int(4u * part) + k, 64);
+    const bool anyTarget = 16u * q < e - s; // whole waves
+
+    if (lane < 16) selfAll[q][lane] = ~0u;
+    uint32_t  queued = 0, masked = 0; // members appended to the queue, and those of them with masks
+    uint32_t  count  = 0;             // this lane's hits
+    uint32_t  listed[Sph ? 1 : 16] = {}; // !Sph: each target's neighbors so far
+    const uint32_t sg     = 4u * g + q;
+    uint32_t*      unions = Sph ? out.unions + size_t(sg) * out.capU : nullptr;
+    // this lane's 16 bits of the masks of a batch
+    uint16_t*      maskAt = Sph ? reinterpret_cast<uint16_t*>(out.masks + (size_t(sg) * out.words + (part >> 1)) * 16 + n) + (part & 1u)
+                                : nullptr;
+
+    // the masks of the next 64 members of the queue (nb of them)
+    auto masks = [&](uint32_t nb) {
+        const uint32_t half = masked & 64u;
+        const float*   A    = que + (half ? NS_QHALF : 0u) + 80u * (n >> 2) + 4u * (n & 3u) + part;
+        floatx4        d[4];
+#pragma unroll
+        for (int m = 0; m < 4; ++m)
+            d[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(A[16 * m], tval, cCol, 0, 0, 0);
+        const uint32_t j = queJ[half + lane];
+        const uint32_t o = selfAll[q][n] - masked;
+        __builtin_amdgcn_sched_barrier(0); // all four in flight before the first result is used
+        // result (m, k): member 16 part + 4 m + k
+        uint32_t P = 0, mn = ~0u;
+#pragma unroll
+        for (int k = 15; k >= 0; --k)
+        {
+            const uint32_t a = __float_as_uint(d[k >> 2][k & 3]);
+            P                = __builtin_amdgcn_alignbit(P, a, 31);
+            mn               = min(mn, a);
+        }
+        if (__builtin_expect(ballot(mn < __float_as_uint(undecided)) != 0, 0))
+        {
+            // the pairs whose FP32 result does not decide, exactly
+            uint32_t amb = 0;
+#pragma unroll
+            for (int k = 15; k >= 0; --k)
+                amb = (amb << 1) | (__float_as_uint(d[k >> 2][k & 3]) < __float_as_uint(undecided) ? 1u : 0u);
+            while (amb)
+            {
+                const uint32_t b = uint32_t(__builtin_ctz(amb));
+                amb &= amb - 1u;
+                if (act && 16u * part + b < nb && exactHit(i, queJ[half + 16u * part + b])) P |= 1u << b;
+            }
+        }
+        // a target is not its own neighbor
+        if ((o >> 4) == part) P &= ~(1u << (o & 15u));
+        count += uint32_t(__builtin_popcount(P));
+        if constexpr (Sph)
+        {
+            if (masked + 64u <= out.capU)
+            {
+                *maskAt = uint16_t(P);
+                if (lane < nb) unions[masked + lane] = j;
+            }
+            maskAt += 64; // two words of 16 targets
+        }
+        else
+        {
+            // reference CPU layout: the k-th hit of target i goes to nbrs[(i - first) * ngmax + k]
+#pragma unroll
+            for (int t = 0; t < 16; ++t)
+            {
+                const uint32_t lo = uint32_t(__builtin_amdgcn_readlane(int(P), t)) |
+                                    (uint32_t(__builtin_amdgcn_readlane(int(P), 16 + t)) << 16);
+                const uint32_t hw = uint32_t(__builtin_amdgcn_readlane(int(P), 32 + t)) |
+                                    (uint32_t(__builtin_amdgcn_readlane(int(P), 48 + t)) << 16);
+                const uint64_t mt = (uint64_t(hw) << 32) | lo;
+                if (mt == 0) continue;
+                const uint32_t pos = listed[t] + rankIn(mt);
+                if (((mt >> lane) & 1u) && nbrs && pos < ngmax)
+                    nbrs[size_t(s + 16u * q + uint32_t(t) - G.first) * ngmax + pos] = j;
+                listed[t] += popc64(mt);
+            }
+        }
+        masked += 64u;
+    };
+
+    // this wave's chunks of the next NS_CHUNKS (their bounds are scalars), loaded a step ahead
+    const uint2* pieces = ranges + size_t(g) * NS_LCAP + NS_PER_WAVE * q;
+    uint32_t     st[NS_PER_WAVE], len[NS_PER_WAVE];
+    double       ax[NS_PER_WAVE], ay[NS_PER_WAVE], az[NS_PER_WAVE];
+    auto         loadChunks = [&](uint32_t k) {
+#pragma unroll
+        for (uint32_t c = 0; c < NS_PER_WAVE; ++c)
+        {
+            const bool  in = k + NS_PER_WAVE * q + c < R;
+            const uint2 v  = in ? pieces[k + c] : make_uint2(0u, 0u);
+            st[c] = v.x, len[c] = v.y - v.x;
+            ax[c] = ay[c] = az[c] = 0.0;
+            if (lane < len[c]) ax[c] = x[st[c] + lane], ay[c] = y[st[c] + lane], az[c] = z[st[c] + lane];
+        }
+    };
+    loadChunks(0u);
+    uint32_t avail = 0, proc = 0;     // entries put into the ring, entries tested
+    uint32_t ringIn = 0, ringOut = 0; // avail and proc modulo the ring's size
+    for (uint32_t fill = 0;; fill += NS_CHUNKS)
+    {
+        const bool last = fill + NS_CHUNKS >= R;
+        float4     ev[NS_PER_WAVE];
+        uint32_t   jv[NS_PER_WAVE];
+        uint64_t   mk[NS_PER_WAVE];
+#pragma unroll
+        for (uint32_t c = 0; c < NS_PER_WAVE; ++c)
+        {
+            double dx = ax[c] - sb.cx, dy = ay[c] - sb.cy, dz = az[c] - sb.cz;
+            if (sb.fold)
+            {
+                dx -= px * rint(dx * box.ilen[0]);
+                dy -= py * rint(dy * box.ilen[1]);
+                dz -= pz * rint(dz * box.ilen[2]);
+            }
+            const float fx = float(dx) * invF, fy = float(dy) * invF, fz = float(dz) * invF;
+            const float ex = fmaxf(fabsf(fx) - sb.hwx, 0.f), ey = fmaxf(fabsf(fy) - sb.hwy, 0.f), ez = fmaxf(fabsf(fz) - sb.hwz, 0.f);
+            mk[c] = ballot(__builtin_fmaf(ez, ez, __builtin_fmaf(ey, ey, ex * ex)) <= sb.lim) &
+                    (len[c] ? ~uint64_t(0) >> (64u - len[c]) : 0u);
+            ev[c]   = make_float4(fx, fy, fz, __builtin_fmaf(fz, fz, __builtin_fmaf(fy, fy, fx * fx)));
+            jv[c]   = st[c] + lane;
+        }
+        if (!last) loadChunks(fill + NS_CHUNKS);
+        uint32_t mine = 0;
+#pragma unroll
+        for (uint32_t c = 0; c < NS_PER_WAVE; ++c)
+            mine += popc64(mk[c]);
+        if (lane == 0) wcnt[q] = mine;
+        __syncthreads(); // the counts; the previous step's batches are tested
+        uint32_t before = 0, total = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k)
+        {
+            const uint32_t v = uint32_t(__builtin_amdgcn_readfirstlane(int(wcnt[k])));
+            before += k < q ? v : 0u;
+            total += v;
+        }
+#pragma unroll
+        for (uint32_t c = 0; c < NS_PER_WAVE; ++c)
+        {
+            if (__builtin_amdgcn_inverse_ballot_w64(mk[c]))
+            {
+                const uint32_t k = before + rankIn(mk[c]);
+                uint32_t       p = ringIn + k;
+                p                = min(p, p - NS_RING);
+                ent[p]           = ev[c];
+                entJ[p]          = jv[c];
+            }
+            before += popc64(mk[c]);
+        }
+        avail += total;
+        ringIn += total;
+        ringIn = ringIn >= NS_RING ? ringIn - NS_RING : ringIn;
+        if (last && q == 3 && lane < ((64u - (avail & 63u)) & 63u))
+        {
+            // pad the last batch
+            uint32_t p = ringIn + lane;
+            p          = min(p, p - NS_RING);
+            ent[p]     = make_float4(0.f, 0.f, 0.f, 1e30f);
+            entJ[p]    = ~0u;
+        }
+        __syncthreads(); // the new entries
+
+        const uint32_t goal = last ? (avail + 63u) & ~63u : avail & ~63u;
+        while (proc < goal && anyTarget)
+        {
+            // 16 targets x 64 entries
+            const float* B = reinterpret_cast<const float*>(ent + ringOut + n) + part;
+            floatx4      d[4];
+#pragma unroll
+            for (int m = 0; m < 4; ++m)
+                d[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(tval, B[64 * m], cRow, 0, 0, 0);
+            const float4   own = ent[ringOut + lane];
+            const uint32_t j = entJ[ringOut + lane], o = j - (s + 16u * q);
+            __builtin_amdgcn_sched_barrier(0);
+            // entry 16 m + n's minimum over the lane's four targets, then over the four parts: the
+            // first swap leaves the lower half with entries of m = 0 and 1, the second each row
+            // of 16 lanes with those of its own m
+            // (as integers: a negative result is below any positive one, and those keep their order)
+            int mn[4];
+#pragma unroll
+            for (int m = 0; m < 4; ++m)
+            {
+                auto bits = [&](int k) { return int(__float_as_uint(d[m][k])); };
+                mn[m]     = min(min(min(bits(0), bits(1)), bits(2)), bits(3));
+            }
+            if (ballot(o < 16u))
+            {
+                // targets among the entries: without their own results
+#pragma unroll
+                for (int m = 0; m < 4; ++m)
+                {
+                    const uint32_t om = entJ[ringOut + 16u * uint32_t(m) + n] - (s + 16u * q) - 4u * part;
+                    mn[m]             = INT_MAX;
+#pragma unroll
+                    for (uint32_t k = 0; k < 4; ++k)
+                        mn[m] = min(mn[m], om == k ? INT_MAX : int(__float_as_uint(d[m][k])));
+                }
+            }
+            const int  a = swapMin<32>(mn[0], mn[2]), b = swapMin<32>(mn[1], mn[3]);
+            const int  v = swapMin<16>(a, b);
+            uint64_t   U = ballot(v < 0);
+            const uint64_t V = ballot(v < int(__float_as_uint(undecided)));
+            if (__builtin_expect(U != V, 0))
+            {
+                // entries whose nearest results do not decide
+                for (uint64_t W = V & ~U; W; W &= W - 1u)
+                {
+                    const uint32_t b  = uint32_t(__builtin_ctzll(W));
+                    const uint32_t jb = uint32_t(__builtin_amdgcn_readlane(int(j), int(b)));
+                    if (ballot(act && i != jb && exactHit(i, jb))) U |= uint64_t(1) << b;
+                }
+            }
+            if (__builtin_amdgcn_inverse_ballot_w64(U))
+            {
+                const uint32_t u = queued + rankIn(U), p = u & 127u;
+                float*         f = que + 4u * (p + 4u * (p >> 4));
+                *reinterpret_cast<float4*>(f) = own;
+                queJ[p]                       = j;
+                if (o < 16u) selfAll[q][o] = u;
+            }
+            queued += popc64(U);
+            proc += 64u;
+            ringOut += 64u;
+            ringOut = ringOut == NS_RING ? 0u : ringOut;
+            waveFence();
+            if (queued - masked >= 64u) masks(64u);
+            waveFence();
+        }
+        proc = goal;
+        if (last) break;
+    }
+    if (masked < queued)
+    {
+        // the rest, padded with members that no target hits
+        const uint32_t nb = queued - masked, p = (masked & 64u) + lane;
+        if (lane >= nb) *reinterpret_cast<float4*>(que + 4u * (p + 4u * (p >> 4))) = make_float4(0.f, 0.f, 0.f, 1e30f);
+        waveFence();
+        masks(nb);
+    }
+    // pair tests of this pass (stored per launched group and summed by nsSumTests: one atomic
+    // per group on a single counter would serialize)
+    if (threadIdx.x == 0) groupTests[blk] = (unsigned long long)avail * (e - s);
+
+    count += uint32_t(__shfl_xor(int(count), 16, 64));
+    count += uint32_t(__shfl_xor(int(count), 32, 64));
+    if constexpr (Sph)
+    {
+        const uint64_t over = ballot(count > ngmax || queued + 64u > out.capU);
+        if (lane == 0) wflag[q] = over != 0;
+        __syncthreads();
+        if (wflag[0] | wflag[1] | wflag[2] | wflag[3])
+        {
+            if (threadIdx.x == 0)
+            {
+                overList[atomicAdd(&flags->overCount, 1u)] = g;
+                groupTests[blk]                            = 0;
+            }
+            return;
+        }
+        if (lane == 0) out.usize[sg] = queued;
+        bool redo = false;
+        if (act && part == 0)
+        {
+            uint32_t ncSph = count + 1;
+            uint32_t ngmin = ng0 / 4;
+            bool     outR  = (ngmin > ncSph) || (ncSph - 1 > ngmax);
+            nc[i] = ncSph; // dataset counts are indexed by particle (sph/find_neighbors.hpp:51)
+            if (outR && iter[i] < 10)
+            {
+                // updateH (sph/kernels.hpp:27-33) in the precision of h, factor from the table
+                Th hn = h[i];
+                if (updateHTab(hfac, ncSph, hn))
+                {
+                    h[i] = hn;
+                    iter[i] += 1;
+                    redo = true;
+                }
+                else
+                    flags->hfacMiss = 1;
+            }
+        }
+        const uint64_t anyRedo = ballot(redo);
+        __syncthreads(); // wflag is read
+        if (lane == 0) wflag[q] = anyRedo != 0;
+        __syncthreads();
+        if (threadIdx.x == 0 && (wflag[0] | wflag[1] | wflag[2] | wflag[3])) redoList[atomicAdd(&flags->redoCount, 1u)] = g;
+    }
+    else
+    {
+        if (act && part == 0) nc[i - G.first] = count;
+    }
+}
+
 __global__ __launch_bounds__(256) void nsInitState(uint8_t* iter, uint32_t first, uint32_t last)
 {
     uint32_t i = first + blockIdx.x * blockDim.x + threadIdx.x;
@@ -644,6 +1150,7 @@ __global__ void nsResetFlags(NsFlags* f, int clearErrors)
     {
         f->redoCount  = 0;
         f->retryCount = 0;
+        f->overCount  = 0;
         f->tests      = 0;
         if (clearErrors)
         {
@@ -792,6 +1299,13 @@ __global__ __launch_bounds__(256) void grpBoundaries(uint32_t first, uint32_t la
 
 // ---------------------------------------------------------------------------
 // host driver shared by both entry points
+static int sumTests(sphx_ctx* ctx, const unsigned long long* gtests, uint32_t n, NsFlags* flags)
+{
+    nsSumTests<<<std::min<uint32_t>(256u, (n + 1023u) / 1024u), 256, 0, ctx->stream>>>(gtests, n, flags);
+    SPHX_LAUNCH_CHECK(ctx, "nsSumTests");
+    return SPHX_OK;
+}
+
 template<class Th, bool Sph>
 static int runSearch(sphx_ctx* ctx, const GroupsDev& G, const double* x, const double* y, const double* z, Th* h,
                      const sphx_box* box, const sphx_octree* t, uint32_t ngmax, uint32_t ng0, uint32_t* nbrs,
@@ -805,8 +1319,11 @@ static int runSearch(sphx_ctx* ctx, const GroupsDev& G, const double* x, const d
     uint32_t* redo   = scratchT<uint32_t>(ctx, S_NS_REDO, 2 * size_t(numG));
     uint32_t* retry  = scratchT<uint32_t>(ctx, S_NS_RETRY, numG);
     auto*     gtests = scratchT<unsigned long long>(ctx, S_NS_TESTS, numG);
+    auto*     gbox   = scratchT<GroupSearch>(ctx, S_NS_BOX, numG);
+    uint32_t* over   = scratchT<uint32_t>(ctx, S_NS_OVER, numG);
     NsFlags*  flags  = scratchT<NsFlags>(ctx, S_SMALL, 1);
-    if (!ranges || !rcnt || !iter || !redo || !retry || !gtests || !flags) return SPHX_ERR_NOMEM;
+    if (!ranges || !rcnt || !iter || !redo || !retry || !gtests || !gbox || !over || !flags)
+        return SPHX_ERR_NOMEM;
     DBox     db = makeDBox(box);
     HFactors hfac;
     if (Sph) SPHX_TRY(hFactors(ctx, ng0, hfac));
@@ -830,7 +1347,7 @@ static int runSearch(sphx_ctx* ctx, const GroupsDev& G, const double* x, const d
             KTimer kt_(ctx, "nsGroupRanges");
             nsGroupRanges<Th><<<numLaunch, 64, 0, ctx->stream>>>(G, list, x, y, z, h, t->childOffsets,
                                                                 t->internalToLeaf, t->layout, t->centers, t->sizes,
-                                                                db, ranges, rcnt, retry, flags);
+                                                                db, ranges, rcnt, gbox, retry, flags);
         }
         SPHX_LAUNCH_CHECK(ctx, "nsGroupRanges");
         {
@@ -838,21 +1355,31 @@ static int runSearch(sphx_ctx* ctx, const GroupsDev& G, const double* x, const d
             uint32_t grid = std::min<uint32_t>(numLaunch, uint32_t(ctx->numCU) * 4u);
             nsGroupRangesRetry<Th><<<grid, 64, 0, ctx->stream>>>(G, x, y, z, h, t->childOffsets, t->internalToLeaf,
                                                                  t->layout, t->centers, t->sizes, db, ranges, rcnt,
-                                                                 retry, flags);
+                                                                 gbox, retry, flags);
         }
         SPHX_LAUNCH_CHECK(ctx, "nsGroupRangesRetry");
         {
             KTimer kt_(ctx, "nsCandidates", true);
-            nsCandidates<Th, Sph><<<numLaunch, 64, 0, ctx->stream>>>(G, list, x, y, z, h, iter, ranges, rcnt, db,
-                                                                    ngmax, ng0, hfac, nbrs, lists, nc, outList,
-                                                                    flags, gtests);
+            nsCandidates<Th, Sph><<<numLaunch, 256, 0, ctx->stream>>>(G, list, x, y, z, h, iter, ranges, rcnt, gbox, db,
+                                                                      ngmax, ng0, hfac, nbrs, lists, nc, outList, over,
+                                                                      flags, gtests);
         }
         SPHX_LAUNCH_CHECK(ctx, "nsCandidates");
-        nsSumTests<<<std::min<uint32_t>(256u, (numLaunch + 1023u) / 1024u), 256, 0, ctx->stream>>>(gtests, numLaunch,
-                                                                                                flags);
-        SPHX_LAUNCH_CHECK(ctx, "nsSumTests");
+        SPHX_TRY(sumTests(ctx, gtests, numLaunch, flags));
         NsFlags hf;
         SPHX_TRY(readBack(ctx, flags, &hf, sizeof(NsFlags)));
+        if (hf.overCount && !hf.overflow && !hf.badGroup)
+        {
+            {
+                KTimer kt_(ctx, "nsCandidatesExact", true);
+                nsCandidatesExact<Th, Sph><<<hf.overCount, 64, 0, ctx->stream>>>(G, over, x, y, z, h, iter, ranges, rcnt,
+                                                                                 db, ngmax, ng0, hfac, nbrs, lists, nc,
+                                                                                 outList, flags, gtests);
+            }
+            SPHX_LAUNCH_CHECK(ctx, "nsCandidatesExact");
+            SPHX_TRY(sumTests(ctx, gtests, hf.overCount, flags));
+            SPHX_TRY(readBack(ctx, flags, &hf, sizeof(NsFlags)));
+        }
         ctx->nsTests += double(hf.tests);
         if (hf.overflow) return fail(ctx, SPHX_ERR_STACK, "neighbor search: traversal capacity exceeded");
         if (hf.badGroup) return argError(ctx, "neighbor search: a target group holds more than 64 particles");

@@ -1,0 +1,123 @@
+"""The neighbor search where its FP32 test can go wrong, against the oracle, bit for bit: ties
+at exactly d = 2h, coincident particles, positions far from the origin, extreme units, radii
+mixed within a group, boxes without a single nearest image, lists cut at ngmax, and particle
+counts around the sizes of quarters, batches and groups."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from tests.helpers import uniform_box
+
+pytestmark = pytest.mark.gpu
+
+CPU = oracle.Cpu("oracle")
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    from sphexa_amd import hydro
+
+    c = hydro.Context(0)
+    yield c
+    c.close()
+
+
+def u32(t):
+    return t.cpu().numpy().view(np.uint32)
+
+
+def dev(a, dtype=torch.float64):
+    return torch.from_numpy(np.ascontiguousarray(a)).to(dtype).to("cuda")
+
+
+def cloud(n, ng=60, periodic=True, lo=0.0, hi=1.0, seed=3):
+    inp, box = uniform_box(n, seed=seed, ng=ng, periodic=periodic, lo=lo, hi=hi)
+    return np.stack([inp["x"], inp["y"], inp["z"]], 1), inp["h"], box
+
+
+def lattice(side, shift, radius_cells):
+    c = (np.arange(side) + shift) / side
+    p = np.stack(np.meshgrid(c, c, c, indexing="ij"), -1).reshape(-1, 3)
+    return p, np.full(len(p), 0.5 * radius_cells / side), oracle.Box.cube(0.0, 1.0, oracle.BC_PERIODIC)
+
+
+def make(case):
+    rng = np.random.default_rng(5)
+    kind, arg = case
+    if kind == "n":
+        return cloud(arg, ng=30, periodic=arg % 2 == 0)
+    if kind == "ties":  # 1/16 cells: exact distances, spheres through many lattice points
+        return lattice(16, 0.5, arg)
+    if kind == "near_ties":  # the same, each distance off by its own rounding
+        return lattice(15, 0.37, arg)
+    if kind == "coincident":
+        p, h, box = cloud(3000)
+        p[1::3] = p[::3]
+        return p, h, box
+    if kind == "offset":
+        return cloud(5000, lo=arg, hi=arg + 1.0)
+    if kind == "units":
+        return cloud(5000, lo=-0.5 * arg, hi=0.5 * arg)
+    if kind == "mixed_h":
+        p, h, box = cloud(5000)
+        return p, h * 10.0 ** rng.uniform(-1.0, 0.4, len(h)), box
+    if kind == "zero_h":
+        p, h, box = cloud(2000)
+        h[rng.random(len(h)) < 0.5] = 0.0
+        return p, h, box
+    if kind == "wide":  # 2h from a fifth of the box to over its half
+        p, h, box = cloud(1500)
+        return p, np.full(len(h), arg), box
+    if kind == "blob":  # one dense blob: groups of few particles beside full ones
+        p = np.clip(0.5 + 0.02 * rng.standard_normal((6000, 3)), 0.0, 1.0)
+        return p, np.full(6000, 0.003), oracle.Box.cube(0.0, 1.0, oracle.BC_OPEN)
+
+
+CASES = [("n", k) for k in (1, 2, 16, 17, 63, 64, 65, 130, 4097)] + [
+    ("ties", 2.0), ("ties", 3.0), ("near_ties", 2.0), ("near_ties", 3.0), ("coincident", 0), ("offset", 1e3),
+    ("offset", 1e8), ("units", 1e-18), ("units", 1e17), ("mixed_h", 0), ("zero_h", 0), ("wide", 0.1), ("wide", 0.2),
+    ("wide", 0.24), ("wide", 0.3), ("blob", 0)]
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: f"{c[0]}-{c[1]}")
+@pytest.mark.parametrize("entry", ["plain", "fp64", "mixed", "cut"])
+def test_search_bit_exact(ctx, case, entry):
+    from sphexa_amd import hydro
+    from sphexa_amd._lib import FP64, MIXED
+
+    print("case search", case, entry, flush=True)
+    p, h, box = make(case)
+    n = len(p)
+    keys = CPU.sfc_keys(*(np.ascontiguousarray(p[:, d]) for d in range(3)), box)
+    keys, order = CPU.sort_by_key(keys, np.arange(n, dtype=np.uint32))
+    x, y, z = (np.ascontiguousarray(p[order, d]) for d in range(3))
+    h = np.ascontiguousarray(h[order])
+    if entry == "mixed":
+        h = h.astype(np.float32).astype(np.float64)
+    gbox = hydro.make_box([box.xmin, box.ymin, box.zmin], [box.xmax, box.ymax, box.zmax], [box.bx, box.by, box.bz])
+    t = hydro.tree_from_keys(ctx, torch.from_numpy(keys.view(np.int64)).to("cuda"), gbox, 64)
+    rt = CPU.tree(keys, box)
+    ngmax = 12 if entry == "cut" else min(n, 3000)
+    ref, ref_nc = CPU.find_neighbors(x, y, z, h, box, rt, ngmax)
+    if entry in ("plain", "cut"):
+        nb, nc = hydro.find_neighbors(ctx, dev(x), dev(y), dev(z), dev(h), gbox, t, ngmax)
+        nb, nc = u32(nb), u32(nc)
+        assert np.array_equal(nc, ref_nc)
+    if entry in ("fp64", "mixed", "cut"):
+        prec = MIXED if entry == "mixed" else FP64
+        ng0 = min(4, ngmax)
+        d = hydro.ParticlesData(n, prec, ng0=ng0, ngmax=ngmax)
+        d.x, d.y, d.z, d.h = dev(x), dev(y), dev(z), dev(h, torch.float32 if prec == MIXED else torch.float64)
+        d.allocate("cuda")
+        hydro.find_neighbors_sfc(ctx, d, gbox, t)
+        if entry == "cut":
+            # the first check is of the plain entry; this one iterates h and keeps the first ngmax
+            assert all(np.array_equal(nb[i, :c], ref[i, :c]) for i, c in enumerate(np.minimum(nc, ngmax)))
+            ref, ref_nc, h = CPU.find_neighbors_sph(x, y, z, h, box, rt, ng0, ngmax)
+            assert np.array_equal(d.h.cpu().numpy(), h)
+            ref_nc = ref_nc - 1
+        nb, nc = u32(hydro.export_neighbors(ctx, d)), u32(d.nc) - 1
+        assert np.array_equal(nc, ref_nc)
+    bad = [i for i, c in enumerate(np.minimum(nc, ngmax)) if not np.array_equal(nb[i, :c], ref[i, :c])]
+    assert not bad, bad[:10]
