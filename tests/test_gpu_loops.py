@@ -75,3 +75,49 @@ def test_fitted_table_loops_equal_table_loops(kind, table, periodic):
             group = next((g for g in GROUPS if f in g), (f,))
             assert err.max().item() < 1e-10 * max(ref[g].abs().max().item() for g in group), f
     assert abs(got["dt"] - ref["dt"]) < 1e-12 * ref["dt"]
+
+
+# The mixed loops' window lists (ORed into LDS for records up to 32 bytes): empty chunks and
+# lists, full chunks and windows, unions of one entry and of several windows, against the
+# FP64-exact loops (one lane per target, no windows) on the same particles.  A wrong or missing
+# slot changes a sum by a whole term; tolerances are those of the other mixed tests (rho, xm,
+# kx 1e-5 relative, IAD 1e-4 of its largest diagonal).
+@pytest.mark.parametrize("n,ng", [(1, 10), (2, 10), (63, 20), (64, 64), (65, 65), (300, 300), (1500, 4), (2000, 30),
+                                  (2000, 1900)])
+@pytest.mark.parametrize("kind", ["std", "ve"])
+def test_mixed_window_lists(kind, n, ng):
+    from sphexa_amd import hydro
+    from sphexa_amd._lib import FP64, MIXED
+
+    print("case lists", kind, n, ng, flush=True)
+    inp, b = uniform_box(n, seed=17, periodic=n < 3, ng=ng)  # (an open box is fitted to the particles: n >= 3)
+    inp = {k: v if k in "xyz" else v.astype(np.float32).astype(np.float64) for k, v in inp.items()}
+    box = hydro.make_box([b.xmin, b.ymin, b.zmin], [b.xmax, b.ymax, b.zmax], [b.bx, b.by, b.bz])
+    out = []
+    for prec in (MIXED, FP64):
+        ctx = hydro.Context(0)
+        try:
+            ctx.set_fp64_exact(True)
+            make = hydro.HydroStep if kind == "std" else hydro.VeHydroStep
+            step = make(ctx, n, box, prec, ng0=4, ngmax=max(4, n))
+            dt = torch.float64 if prec == FP64 else torch.float32
+            d_inp = {k: torch.from_numpy(np.ascontiguousarray(v)).to("cuda", torch.float64 if k in "xyz" else dt)
+                     for k, v in inp.items()}
+            if kind == "ve":
+                d_inp["alpha"] = torch.full((n,), 0.25, dtype=dt, device="cuda")
+            step.compute_forces(d_inp)
+            out.append({f: field(step, f) for f in (("rho", "c11", "c22", "c33") if kind == "std" else ("xm", "kx"))})
+            out[-1]["nc"] = step.d.nc.clone()
+        finally:
+            ctx.close()
+    got, ref = out
+    assert torch.equal(got["nc"], ref["nc"])
+    for f in POSITIVE:
+        if f in got:
+            assert ((got[f] - ref[f]).abs() <= 1e-5 * ref[f]).all(), f
+    # the IAD inverts its sums; compared where they are well determined
+    well = ref["nc"] > 30
+    if kind == "std" and well.any():
+        scale = max(ref[f][well].abs().max().item() for f in ("c11", "c22", "c33"))
+        for f in ("c11", "c22", "c33"):
+            assert ((got[f] - ref[f])[well].abs() <= 1e-4 * scale).all(), f
