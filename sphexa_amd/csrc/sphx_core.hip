@@ -222,7 +222,7 @@ int exclusiveScanU32(sphx_ctx* ctx, const uint32_t* in, uint32_t* out, uint64_t 
 // ===========================================================================
 // LSD radix sort, 8-bit digits.  Per pass: tile histograms -> per-digit scan over the
 // tiles -> stable scatter through an LDS-staged local sort so that global writes are
-// contiguous runs per digit.  Three launches per pass: the digit-major histogram is
+// contiguous runs per digit.  Three launches per pass (two for few tiles): the digit-major histogram is
 // scanned one column (digit) per block, and each scatter tile adds the exclusive scan
 // of the 256 digit totals itself.
 constexpr int SORT_THREADS = 256;
@@ -321,7 +321,9 @@ __global__ __launch_bounds__(256) void radixVaryingBits(const uint64_t* __restri
                     (part[1][0] & part[1][1] & part[1][2] & part[1][3]);
 }
 
-template<bool HasVals>
+// ColumnScan: tileOfs holds the tiles' counts as radixUpsweep left them, and every tile sums its
+// digits' columns itself (few tiles: a launch less per pass)
+template<bool HasVals, bool ColumnScan>
 __global__ __launch_bounds__(SORT_THREADS) void radixScatter(const uint64_t* __restrict__ kin,
                                                              const uint32_t* __restrict__ vin,
                                                              uint64_t* __restrict__ kout, uint32_t* __restrict__ vout,
@@ -389,9 +391,26 @@ __global__ __launch_bounds__(SORT_THREADS) void radixScatter(const uint64_t* __r
         uint32_t start = blockExclusiveScan256(tot, sWave, total);
         // the digit's first output position: the totals of the smaller digits plus the
         // counts of this digit in the tiles before this one
-        uint32_t below = blockExclusiveScan256(tileOfs[uint64_t(RADIX) * numTiles + d], sWave, all);
+        uint32_t before = 0, digits = 0;
+        if constexpr (ColumnScan)
+        {
+            const uint32_t* col = tileOfs + d * numTiles;
+#pragma unroll 8
+            for (uint32_t t = 0; t < numTiles; ++t)
+            {
+                const uint32_t c = col[t];
+                digits += c;
+                before += t < blockIdx.x ? c : 0u;
+            }
+        }
+        else
+        {
+            digits = tileOfs[uint64_t(RADIX) * numTiles + d];
+            before = tileOfs[uint64_t(d) * numTiles + blockIdx.x];
+        }
+        uint32_t below = blockExclusiveScan256(digits, sWave, all);
         dStart[d]      = start;
-        gOfs[d]        = below + tileOfs[uint64_t(d) * numTiles + blockIdx.x];
+        gOfs[d]        = below + before;
     }
     __syncthreads();
 
@@ -429,6 +448,145 @@ __global__ void copyKV(const uint64_t* ks, const uint32_t* vs, uint64_t* kd, uin
     }
 }
 
+// The whole sort of up to BLOCK_SORT_MAX keys in one workgroup: keys and values stay in
+// registers and move through LDS once per pass; passes over digits that no two keys differ in
+// are skipped.  Same ranks as radixScatter, so the same stable order.  Launches bound the small
+// sorts (three per pass, and a host read): eight passes over 1,000 / 4,096 / 10,000 keys with
+// values took 100 / 120 / 126 us, here 40 / 54 / 91.
+constexpr int BLOCK_SORT_THREADS = 1024, BLOCK_SORT_WAVES = BLOCK_SORT_THREADS / 64;
+constexpr int BLOCK_SORT_ITEMS   = 11; // as many keys and values as LDS holds
+constexpr int BLOCK_SORT_MAX = BLOCK_SORT_THREADS * BLOCK_SORT_ITEMS;
+template<bool HasVals>
+__global__ __launch_bounds__(BLOCK_SORT_THREADS) void radixSortBlock(uint64_t* __restrict__ keys,
+                                                                     uint32_t* __restrict__ vals, uint32_t n,
+                                                                     int firstShift, int keyBits)
+{
+    __shared__ uint64_t sk[BLOCK_SORT_MAX];
+    __shared__ uint32_t sv[HasVals ? BLOCK_SORT_MAX : 1];
+    __shared__ uint32_t wcount[BLOCK_SORT_WAVES][RADIX];
+    __shared__ uint32_t dStart[RADIX];
+    __shared__ uint32_t sWave[4];
+    __shared__ uint64_t part[2][BLOCK_SORT_WAVES];
+
+    const unsigned lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const uint32_t base   = wave * 64u * BLOCK_SORT_ITEMS + lane; // item k: element base + 64 k
+    const uint64_t ltMask = (uint64_t(1) << lane) - 1;
+
+    uint64_t key[BLOCK_SORT_ITEMS], o = 0, a = ~uint64_t(0);
+    uint32_t val[BLOCK_SORT_ITEMS], rank[BLOCK_SORT_ITEMS];
+#pragma unroll
+    for (int k = 0; k < BLOCK_SORT_ITEMS; ++k)
+    {
+        const uint32_t i = base + 64u * uint32_t(k);
+        key[k]           = i < n ? keys[i] : 0;
+        if constexpr (HasVals) val[k] = i < n ? vals[i] : 0;
+        if (i < n) o |= key[k], a &= key[k];
+    }
+    for (int s = 32; s > 0; s >>= 1)
+        o |= __shfl_xor(o, s, 64), a &= __shfl_xor(a, s, 64);
+    if (lane == 0) part[0][wave] = o, part[1][wave] = a;
+    __syncthreads();
+    o = 0, a = ~uint64_t(0);
+    for (int w = 0; w < BLOCK_SORT_WAVES; ++w)
+        o |= part[0][w], a &= part[1][w];
+    const uint64_t varies = o ^ a;
+
+    for (int shift = firstShift; shift < keyBits; shift += 8)
+    {
+        if (((varies >> shift) & 0xFFull) == 0) continue;
+        for (unsigned d = threadIdx.x; d < BLOCK_SORT_WAVES * RADIX; d += BLOCK_SORT_THREADS)
+            (&wcount[0][0])[d] = 0;
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < BLOCK_SORT_ITEMS; ++k)
+        {
+            const bool valid = base + 64u * uint32_t(k) < n;
+            unsigned   d     = unsigned(key[k] >> shift) & 255u;
+            uint64_t   peers = __ballot(valid);
+            if (peers == 0) break; // the wave's later items lie beyond n too
+#pragma unroll
+            for (int b = 0; b < 8; ++b)
+            {
+                bool     bit = (d >> b) & 1u;
+                uint64_t bb  = __ballot(bit);
+                peers &= bit ? bb : ~bb;
+            }
+            unsigned below = unsigned(__popcll(peers & ltMask));
+            unsigned cnt   = unsigned(__popcll(peers));
+            uint32_t old   = valid ? wcount[wave][d] : 0u;
+            rank[k]        = old + below;
+            __builtin_amdgcn_wave_barrier();
+            if (valid && below == 0) wcount[wave][d] = old + cnt;
+            __builtin_amdgcn_wave_barrier();
+        }
+        __syncthreads();
+        // per digit: exclusive offsets across waves, and the digit's start
+        uint32_t tot = 0;
+        if (threadIdx.x < RADIX)
+        {
+            uint32_t c[BLOCK_SORT_WAVES];
+#pragma unroll
+            for (int w = 0; w < BLOCK_SORT_WAVES; ++w)
+                c[w] = wcount[w][threadIdx.x];
+#pragma unroll
+            for (int w = 0; w < BLOCK_SORT_WAVES; ++w)
+            {
+                wcount[w][threadIdx.x] = tot;
+                tot += c[w];
+            }
+        }
+        // exclusive scan of the 256 totals (4 waves)
+        uint32_t in = tot;
+        for (int s = 1; s < 64; s <<= 1)
+        {
+            const uint32_t v = uint32_t(__shfl_up(int(in), s, 64));
+            if (lane >= unsigned(s)) in += v;
+        }
+        if (lane == 63 && wave < 4) sWave[wave] = in;
+        __syncthreads();
+        if (threadIdx.x < RADIX)
+        {
+            uint32_t start = in - tot;
+            for (unsigned w = 0; w < wave; ++w)
+                start += sWave[w];
+            dStart[threadIdx.x] = start;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < BLOCK_SORT_ITEMS; ++k)
+        {
+            if (base + 64u * uint32_t(k) < n)
+            {
+                const unsigned d   = unsigned(key[k] >> shift) & 255u;
+                const uint32_t pos = dStart[d] + wcount[wave][d] + rank[k];
+                sk[pos]            = key[k];
+                if constexpr (HasVals) sv[pos] = val[k];
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < BLOCK_SORT_ITEMS; ++k)
+        {
+            const uint32_t i = base + 64u * uint32_t(k);
+            if (i < n)
+            {
+                key[k] = sk[i];
+                if constexpr (HasVals) val[k] = sv[i];
+            }
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < BLOCK_SORT_ITEMS; ++k)
+    {
+        const uint32_t i = base + 64u * uint32_t(k);
+        if (i < n)
+        {
+            keys[i] = key[k];
+            if constexpr (HasVals) vals[i] = val[k];
+        }
+    }
+}
+
 // Work buffers of one sort: ping-pong keys and values (n each) and the per-tile digit
 // histograms followed by the digit totals (RADIX * (tiles + 1)).
 struct SortWork
@@ -437,6 +595,11 @@ struct SortWork
     uint32_t* vAlt;
     uint32_t* hist;
 };
+
+// Up to this many tiles the scatter sums the digits' columns itself instead of a launch in
+// between.  Eight passes, separate / fused: 27,000 keys (18 tiles) 126 / 106 us, 60,000 (40)
+// 127 / 113, 100,000 (66) 128 / 124, 200,000 (131) 133 / 153.
+constexpr uint32_t kFusedScanTiles = 64;
 
 // One pass over the 8-bit digit at `shift`: (kSrc, vSrc) -> (kDst, vDst), stable.
 // tileVar != nullptr: the histogram kernel also writes each tile's OR and AND of the keys.
@@ -448,16 +611,17 @@ static int radixPass(sphx_ctx* ctx, sphx_ctx* tctx, const uint64_t* kSrc, const 
         radixUpsweep<<<numTiles, SORT_THREADS, 0, ctx->stream>>>(kSrc, n, shift, hist, numTiles, tileVar);
     }
     SPHX_LAUNCH_CHECK(ctx, "radixUpsweep");
-    radixColumnScan<<<RADIX, 256, 0, ctx->stream>>>(hist, numTiles);
-    SPHX_LAUNCH_CHECK(ctx, "radixColumnScan");
+    const bool fused = numTiles <= kFusedScanTiles;
+    if (!fused)
+    {
+        radixColumnScan<<<RADIX, 256, 0, ctx->stream>>>(hist, numTiles);
+        SPHX_LAUNCH_CHECK(ctx, "radixColumnScan");
+    }
     {
         KTimer kt_(tctx, "radixScatter");
-        if (vSrc)
-            radixScatter<true><<<numTiles, SORT_THREADS, 0, ctx->stream>>>(kSrc, vSrc, kDst, vDst, n, shift, hist,
-                                                                          numTiles);
-        else
-            radixScatter<false><<<numTiles, SORT_THREADS, 0, ctx->stream>>>(kSrc, nullptr, kDst, nullptr, n, shift,
-                                                                           hist, numTiles);
+        auto   scatter = vSrc ? (fused ? radixScatter<true, true> : radixScatter<true, false>)
+                              : (fused ? radixScatter<false, true> : radixScatter<false, false>);
+        scatter<<<numTiles, SORT_THREADS, 0, ctx->stream>>>(kSrc, vSrc, kDst, vSrc ? vDst : nullptr, n, shift, hist, numTiles);
     }
     SPHX_LAUNCH_CHECK(ctx, "radixScatter");
     return SPHX_OK;
@@ -476,6 +640,16 @@ static int radixSortWith(sphx_ctx* ctx, uint64_t* keys, uint32_t* vals, uint64_t
 {
     if (n <= 1) return SPHX_OK;
     if (n >= (uint64_t(1) << 32)) return argError(ctx, "sort: n must be < 2^32");
+    if (n <= BLOCK_SORT_MAX)
+    {
+        const int firstShift = 8 * (lowBits / 8);
+        KTimer    kt_(own ? nullptr : ctx, "radixSortBlock");
+        if (vals) radixSortBlock<true><<<1, BLOCK_SORT_THREADS, 0, ctx->stream>>>(keys, vals, uint32_t(n), firstShift, keyBits);
+        else radixSortBlock<false><<<1, BLOCK_SORT_THREADS, 0, ctx->stream>>>(keys, nullptr, uint32_t(n), firstShift, keyBits);
+        kt_.stop();
+        SPHX_LAUNCH_CHECK(ctx, "radixSortBlock");
+        return SPHX_OK;
+    }
     uint32_t numTiles = uint32_t((n + SORT_TILE - 1) / SORT_TILE);
 
     uint64_t* kAlt;
@@ -558,7 +732,10 @@ int radixSortPairs(sphx_ctx* ctx, uint64_t* keys, uint32_t* vals, uint64_t n, in
 // four prefix passes the next kPrefixRetryCalls sorts of the context run them directly,
 // after three the next sort takes four.
 constexpr uint32_t kRunMax           = 64;
-constexpr uint64_t kPrefixSortMinN   = uint64_t(1) << 18;
+// The prefix sort starts where the sort in one workgroup stops being the faster one (us, Hilbert
+// keys with values, one workgroup / prefix): 4,096 54 / 60, 6,000 60 / 60, 8,000 74 / 60.  Eight
+// passes took 125 us there and 131 at 100,000 keys, where the prefix sort takes 65.
+constexpr uint64_t kPrefixSortMinN   = 6144;
 constexpr int      kPrefixRetryCalls = 16;
 constexpr uint32_t kFixOwned = 192; // positions written per wave
 constexpr uint32_t kFixWin   = 256; // the wave's window: 4 keys per lane
