@@ -205,6 +205,7 @@ struct sphx_ctx
     // pinned host staging for small device-to-host reads (kHostStageBytes; nullptr: pageable
     // reads) and the event that marks a started read
     void*      hostStage = nullptr;
+    uint32_t   readSeq   = 0; // the last read's number, which its kernel leaves in the staging's flag
     hipEvent_t readEvent = nullptr;
     // deferred Courant time step (SPHX_OPT_DEFER_MIN_DT): the momentum-energy entries copy
     // the reduced minimum into minDtHost (pinned) and record minDtEvent; sphx_min_dt_courant
@@ -221,8 +222,8 @@ namespace sphx
 
 int fail(sphx_ctx* ctx, int code, const std::string& msg);
 
-// Small device-to-host reads through the context's pinned staging buffer.  readBack copies
-// bytes from src and waits for the stream; readBackStart enqueues the copy and marks it
+// Small device-to-host reads through the context's pinned staging buffer.  readBack brings
+// bytes from src and waits for them and all work before; readBackStart enqueues the copy and marks it
 // with an event, and readBackFinish waits for that copy alone (work enqueued after the
 // start keeps running) and delivers the bytes.  One started read at a time.
 constexpr size_t kHostStageBytes = 4096;
