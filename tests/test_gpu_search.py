@@ -72,12 +72,16 @@ def make(case):
     if kind == "blob":  # one dense blob: groups of few particles beside full ones
         p = np.clip(0.5 + 0.02 * rng.standard_normal((6000, 3)), 0.0, 1.0)
         return p, np.full(6000, 0.003), oracle.Box.cube(0.0, 1.0, oracle.BC_OPEN)
+    if kind == "levels":  # density ~ r^-2: a group's candidate leaves are of many levels, and hundreds
+        d = rng.standard_normal((20000, 3))
+        r = 0.499 * rng.random((20000, 1))
+        return 0.5 + r * d / np.linalg.norm(d, axis=1, keepdims=True), np.full(20000, arg), oracle.Box.cube(0.0, 1.0)
 
 
 CASES = [("n", k) for k in (1, 2, 16, 17, 63, 64, 65, 130, 4097)] + [
     ("ties", 2.0), ("ties", 3.0), ("near_ties", 2.0), ("near_ties", 3.0), ("coincident", 0), ("offset", 1e3),
     ("offset", 1e8), ("units", 1e-18), ("units", 1e17), ("mixed_h", 0), ("zero_h", 0), ("wide", 0.1), ("wide", 0.2),
-    ("wide", 0.24), ("wide", 0.3), ("blob", 0)]
+    ("wide", 0.24), ("wide", 0.3), ("blob", 0), ("levels", 0.005), ("levels", 0.03)]
 
 
 @pytest.mark.parametrize("case", CASES, ids=lambda c: f"{c[0]}-{c[1]}")
