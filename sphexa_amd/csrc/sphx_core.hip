@@ -996,7 +996,10 @@ __global__ __launch_bounds__(256) void gatherKernel(const uint32_t* __restrict__
 }
 
 // several arrays permuted by one ordering: order[i] is read once, every array's element
-// is loaded before any is stored (the loads overlap in flight)
+// is loaded before any is stored (the loads overlap in flight).  Neighboring outputs come from
+// nearby inputs, so the blocks go to the XCDs in contiguous ranges and share their lines in L2:
+// lattice order to SFC order at 256^3, 0.71 -> 0.68 ms (FP64 0.81 -> 0.76), 128^3 0.114 -> 0.103;
+// a random order is bound by its sectors either way (4 M: 0.72).
 struct GatherSet
 {
     const void* in[SPHX_GATHER_MAX_ARRAYS];
@@ -1007,7 +1010,7 @@ struct GatherSet
 
 __global__ __launch_bounds__(256) void gatherArraysKernel(const uint32_t* __restrict__ order, GatherSet s, uint64_t n)
 {
-    uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    uint64_t i = uint64_t(xcdContiguous(blockIdx.x, gridDim.x)) * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const uint32_t j = order[i];
     uint64_t       v[SPHX_GATHER_MAX_ARRAYS];
