@@ -125,9 +125,10 @@ def test_mixed_window_lists(kind, n, ng):
 
 @pytest.mark.parametrize("clean", [False, True])
 @pytest.mark.parametrize("length", [1e-3, 1.0, 1e3])
-def test_mixed_ve_pairs(length, clean):
-    """Mixed VE pairs with 1/h^3 in the records and no square root, in units of h from 1e-4 to 100 and
-    with coincident particles (r = 0), against the FP64 loops; the mixed mode's tolerances."""
+def test_ve_pairs(length, clean):
+    """VE pairs with a reciprocal square root for the division by |r| and (mixed) 1/h^3 in the records, in
+    units of h from 1e-4 to 100 and with coincident particles (r = 0), against the FP64-exact loops.
+    Mixed: the mode's tolerances; FP64: the suite's 1e-10, times 10 for the poles of prho (gradh = 0)."""
     from sphexa_amd import hydro
     from sphexa_amd._lib import FP64, MIXED
 
@@ -140,9 +141,10 @@ def test_mixed_ve_pairs(length, clean):
     inp = {k: v if k in "xyz" else v.astype(np.float32).astype(np.float64) for k, v in inp.items()}
     box = hydro.make_box([b.xmin, b.ymin, b.zmin], [b.xmax, b.ymax, b.zmax], [b.bx, b.by, b.bz])
     out = []
-    for prec in (MIXED, FP64):
+    for prec, exact in ((MIXED, False), (FP64, False), (FP64, True)):
         ctx = hydro.Context(0)
         try:
+            ctx.set_fp64_exact(exact)
             step = hydro.VeHydroStep(ctx, n, box, prec, grad_v=True, av_clean=clean, ng0=100)
             d_inp = {k: torch.from_numpy(np.ascontiguousarray(v)).to("cuda", torch.float64 if k in "xyz" else step.d.dtype)
                      for k, v in inp.items()}
@@ -152,7 +154,8 @@ def test_mixed_ve_pairs(length, clean):
         finally:
             ctx.close()
         out[-1]["minDt"] = torch.tensor(dt, dtype=torch.float64)
-    got, ref = out
-    for f in ref:
-        scale = max(ref[k].abs().max() for k in GROUPS[0]) if f in GROUPS[0] else ref[f].abs().max()
-        assert ((got[f] - ref[f]).abs() <= 2e-3 * scale).all(), f
+    ref = out.pop()
+    for got, tol in zip(out, (2e-3, 1e-9)):
+        for f in ref:
+            scale = max(ref[k].abs().max() for k in GROUPS[0]) if f in GROUPS[0] else ref[f].abs().max()
+            assert ((got[f] - ref[f]).abs() <= tol * scale).all(), (f, tol)
