@@ -277,7 +277,7 @@ def roofline(kernels, pairs, n, steps, precision, tests):
             "frac": (achieved / peak) if achieved else None, "traffic": None, "per_launch_ms": per_launch_ms,
             "launches": launches, "work": unit_note,
             "peak_note": "MI355X published vector peak for the kernel's arithmetic (FP64 78.6 for the "
-                         "neighbor search and the FP64 loops, FP32 157.3 for the mixed loops); MFMA is not used"}
+                         "neighbor search and the FP64 loops, FP32 157.3 for the mixed loops); MFMA runs only the search's distance tests"}
 
 
 def measured_traffic(kernel, workload_tag):
