@@ -44,6 +44,21 @@ struct NsFlags
     uint32_t           overCount;  // groups that nsCandidates leaves to nsCandidatesExact
 };
 
+// minimum and maximum over the wave's numbers, the same in every lane: a NaN (of a particle without a
+// usable position or h) is left out
+__device__ inline double waveMinNumber(double v)
+{
+    for (int o = 32; o > 0; o >>= 1)
+        v = fmin(v, __shfl_xor(v, o, 64));
+    return v;
+}
+__device__ inline double waveMaxNumber(double v)
+{
+    for (int o = 32; o > 0; o >>= 1)
+        v = fmax(v, __shfl_xor(v, o, 64));
+    return v;
+}
+
 __device__ inline bool nodeOverlapsBox(const double* __restrict__ centers, const double* __restrict__ sizes, int node,
                                        const double gc[3], const double gh[3], const DBox& box)
 {
@@ -149,11 +164,11 @@ __device__ void groupRangesOf(uint32_t g, GroupsDev G, const double* __restrict_
 #pragma unroll
         for (int d = 0; d < 3; ++d)
         {
-            lo[d] = waveMin(act ? px[d] - r : INFINITY);
-            hi[d] = waveMax(act ? px[d] + r : -INFINITY);
+            lo[d] = waveMinNumber(act ? px[d] - r : INFINITY);
+            hi[d] = waveMaxNumber(act ? px[d] + r : -INFINITY);
         }
-        rmin = waveMin(act ? r : INFINITY);
-        rmax = waveMax(act ? r : -INFINITY);
+        rmin = waveMinNumber(act ? r : INFINITY);
+        rmax = waveMaxNumber(act ? r : -INFINITY);
     }
     if (!(lo[0] <= hi[0]))
     {

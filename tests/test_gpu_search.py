@@ -125,3 +125,61 @@ def test_search_bit_exact(ctx, case, entry):
         assert np.array_equal(nc, ref_nc)
     bad = [i for i, c in enumerate(np.minimum(nc, ngmax)) if not np.array_equal(nb[i, :c], ref[i, :c])]
     assert not bad, bad[:10]
+
+
+def not_a_number(n, rng):
+    """Particles whose values a test replaces: first, middle and last lanes of groups and quarters, a whole
+    group, some at random; half of their NaN have the sign bit."""
+    bad = np.zeros(n, bool)
+    bad[[0, 5, 64 + 15, 64 + 16, 128 + 63, 192]] = True
+    bad[256:320] = True
+    bad |= rng.random(n) < 0.02
+    nan = np.where(rng.random(n) < 0.5, np.nan, -np.nan)
+    return bad, nan
+
+
+def search_both(ctx, x, y, z, h, box, keys, entry, ngmax, ng0=4):
+    """(lists, counts) of the device, of the oracle, for sorted particles with a tree from `keys`."""
+    from sphexa_amd import hydro
+    from sphexa_amd._lib import FP64, MIXED
+
+    n = len(x)
+    gbox = hydro.make_box([box.xmin, box.ymin, box.zmin], [box.xmax, box.ymax, box.zmax], [box.bx, box.by, box.bz])
+    t = hydro.tree_from_keys(ctx, torch.from_numpy(keys.view(np.int64)).to("cuda"), gbox, 64)
+    ref, ref_nc = CPU.find_neighbors(x, y, z, h, box, CPU.tree(keys, box), ngmax)
+    if entry == "plain":
+        nb, nc = hydro.find_neighbors(ctx, dev(x), dev(y), dev(z), dev(h), gbox, t, ngmax)
+        return u32(nb), u32(nc), ref, ref_nc
+    prec = MIXED if entry == "mixed" else FP64
+    d = hydro.ParticlesData(n, prec, ng0=ng0, ngmax=ngmax)
+    d.x, d.y, d.z, d.h = dev(x), dev(y), dev(z), dev(h, torch.float32 if prec == MIXED else torch.float64)
+    d.allocate("cuda")
+    hydro.find_neighbors_sfc(ctx, d, gbox, t)
+    return u32(hydro.export_neighbors(ctx, d)), u32(d.nc) - 1, ref, ref_nc
+
+
+def sorted_cloud(n, entry, **kw):
+    p, h, box = cloud(n, **kw)
+    keys, order = CPU.sort_by_key(CPU.sfc_keys(*(np.ascontiguousarray(p[:, d]) for d in range(3)), box),
+                                  np.arange(n, dtype=np.uint32))
+    x, y, z = (np.ascontiguousarray(p[order, d]) for d in range(3))
+    h = h[order]
+    return x, y, z, h.astype(np.float32).astype(np.float64) if entry == "mixed" else h, box, keys
+
+
+def assert_same_lists(which, nb, nc, ref, ref_nc):
+    assert np.array_equal(nc[which], ref_nc[which])
+    bad = [i for i in np.flatnonzero(which) if not np.array_equal(nb[i, :nc[i]], ref[i, :nc[i]])]
+    assert not bad, bad[:10]
+
+
+@pytest.mark.parametrize("n", [60, 3000])  # a tree of one leaf, leaves of several levels
+@pytest.mark.parametrize("entry", ["plain", "fp64", "mixed"])
+def test_neighbors_of_targets_beside_nan_smoothing_lengths(ctx, entry, n):
+    """A target with h = NaN leaves the lists of its group's other targets as they are."""
+    print("case nan h", entry, n, flush=True)
+    x, y, z, h, box, keys = sorted_cloud(n, entry, ng=40)
+    bad, nan = not_a_number(3000, np.random.default_rng(2))
+    bad, nan = bad[:n], nan[:n]
+    h[bad] = nan[bad]
+    assert_same_lists(~bad, *search_both(ctx, x, y, z, h, box, keys, entry, min(n, 400)))
