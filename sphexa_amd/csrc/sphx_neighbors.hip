@@ -859,8 +859,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void n
         return dx * dx + dy * dy + dz * dz < 4.0 * hi * hi;
     };
 
-    // MFMA operand of the targets and C; a target without neighbors (none, or not finite)
-    // gets +1e30 for every distance
+    // MFMA operand of the targets and C; a target without neighbors (none, or a position or h that
+    // is no number) gets +1e30 for every distance
     float tx = 4.f, ty = 4.f, tz = 4.f, r2 = 0.f;
     if (act)
     {
@@ -869,7 +869,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void n
         r2 = float(rs * rs);
     }
     const float undecided = sb.undecided;
-    const bool  usable = fabsf(tx) <= 2.f && fabsf(ty) <= 2.f && fabsf(tz) <= 2.f;
+    const bool  usable = fabsf(tx) <= 2.f && fabsf(ty) <= 2.f && fabsf(tz) <= 2.f && r2 == r2; // (false for NaN)
     const float tval   = part == 3 ? 1.f : !usable ? 0.f : -2.f * (part == 0 ? tx : part == 1 ? ty : tz);
     const float c0     = usable ? tx * tx + ty * ty + tz * tz - r2 + 0.5f * undecided : 1e30f;
     const floatx4 cCol = {c0, c0, c0, c0};

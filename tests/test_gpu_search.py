@@ -183,3 +183,15 @@ def test_neighbors_of_targets_beside_nan_smoothing_lengths(ctx, entry, n):
     bad, nan = bad[:n], nan[:n]
     h[bad] = nan[bad]
     assert_same_lists(~bad, *search_both(ctx, x, y, z, h, box, keys, entry, min(n, 400)))
+
+
+@pytest.mark.parametrize("entry", ["plain", "fp64", "mixed"])
+def test_targets_with_nan_smoothing_lengths_have_no_neighbors(ctx, entry):
+    """h = NaN, of either sign: d^2 < (2h)^2 holds for no candidate."""
+    print("case nan h targets", entry, flush=True)
+    x, y, z, h, box, keys = sorted_cloud(3000, entry, ng=40)
+    bad, nan = not_a_number(3000, np.random.default_rng(2))
+    h[bad] = nan[bad]
+    nb, nc, ref, ref_nc = search_both(ctx, x, y, z, h, box, keys, entry, 400)
+    assert not ref_nc[bad].any()
+    assert_same_lists(np.ones(3000, bool), nb, nc, ref, ref_nc)
