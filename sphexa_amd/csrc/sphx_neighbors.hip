@@ -992,9 +992,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void n
             }
             const float fx = float(dx) * invF, fy = float(dy) * invF, fz = float(dz) * invF;
             const float ex = fmaxf(fabsf(fx) - sb.hwx, 0.f), ey = fmaxf(fabsf(fy) - sb.hwy, 0.f), ez = fmaxf(fabsf(fz) - sb.hwz, 0.f);
-            mk[c] = ballot(__builtin_fmaf(ez, ez, __builtin_fmaf(ey, ey, ex * ex)) <= sb.lim) &
+            const float e2 = __builtin_fmaf(fz, fz, __builtin_fmaf(fy, fy, fx * fx));
+            // (fmaxf drops a NaN coordinate, |e|^2 keeps it)
+            mk[c] = ballot(__builtin_fmaf(ez, ez, __builtin_fmaf(ey, ey, ex * ex)) <= sb.lim) & ballot(e2 == e2) &
                     (len[c] ? ~uint64_t(0) >> (64u - len[c]) : 0u);
-            ev[c]   = make_float4(fx, fy, fz, __builtin_fmaf(fz, fz, __builtin_fmaf(fy, fy, fx * fx)));
+            ev[c]   = make_float4(fx, fy, fz, e2);
             jv[c]   = st[c] + lane;
         }
         if (!last) loadChunks(fill + NS_CHUNKS);

@@ -195,3 +195,18 @@ def test_targets_with_nan_smoothing_lengths_have_no_neighbors(ctx, entry):
     nb, nc, ref, ref_nc = search_both(ctx, x, y, z, h, box, keys, entry, 400)
     assert not ref_nc[bad].any()
     assert_same_lists(np.ones(3000, bool), nb, nc, ref, ref_nc)
+
+
+@pytest.mark.parametrize("periodic", [False, True])
+@pytest.mark.parametrize("entry", ["plain", "fp64", "mixed"])
+def test_particles_with_nan_positions_are_no_neighbors(ctx, entry, periodic):
+    """A NaN coordinate, of either sign, in the tree's range of some leaf: no target's neighbor, and none itself."""
+    print("case nan positions", entry, periodic, flush=True)
+    x, y, z, h, box, keys = sorted_cloud(3000, entry, ng=40, periodic=periodic)
+    bad, nan = not_a_number(3000, np.random.default_rng(4))
+    for d, a in enumerate((x, y, z)):
+        some = np.flatnonzero(bad)[d::3]
+        a[some] = nan[some]
+    nb, nc, ref, ref_nc = search_both(ctx, x, y, z, h, box, keys, entry, 400)
+    assert not ref_nc[bad].any()
+    assert_same_lists(np.ones(3000, bool), nb, nc, ref, ref_nc)
