@@ -991,12 +991,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void n
                 dz -= pz * rint(dz * box.ilen[2]);
             }
             const float fx = float(dx) * invF, fy = float(dy) * invF, fz = float(dz) * invF;
-            const float ex = fmaxf(fabsf(fx) - sb.hwx, 0.f), ey = fmaxf(fabsf(fy) - sb.hwy, 0.f), ez = fmaxf(fabsf(fz) - sb.hwz, 0.f);
-            const float e2 = __builtin_fmaf(fz, fz, __builtin_fmaf(fy, fy, fx * fx));
-            // (fmaxf drops a NaN coordinate, |e|^2 keeps it)
-            mk[c] = ballot(__builtin_fmaf(ez, ez, __builtin_fmaf(ey, ey, ex * ex)) <= sb.lim) & ballot(e2 == e2) &
+            // the distance from the box; |f| - min(|f|, hw) stays NaN for a NaN coordinate, which is no
+            // neighbor (max(|f| - hw, 0) would be 0)
+            const float ex = fabsf(fx) - fminf(fabsf(fx), sb.hwx), ey = fabsf(fy) - fminf(fabsf(fy), sb.hwy),
+                        ez = fabsf(fz) - fminf(fabsf(fz), sb.hwz);
+            mk[c] = ballot(__builtin_fmaf(ez, ez, __builtin_fmaf(ey, ey, ex * ex)) <= sb.lim) &
                     (len[c] ? ~uint64_t(0) >> (64u - len[c]) : 0u);
-            ev[c]   = make_float4(fx, fy, fz, e2);
+            ev[c]   = make_float4(fx, fy, fz, __builtin_fmaf(fz, fz, __builtin_fmaf(fy, fy, fx * fx)));
             jv[c]   = st[c] + lane;
         }
         if (!last) loadChunks(fill + NS_CHUNKS);
