@@ -92,18 +92,22 @@ struct GroupSearch
 __device__ inline GroupSearch groupSearch(const double gc[3], const double gh[3], double rmin, double rmax, const DBox& box,
                                           bool exact)
 {
-    // candidates are folded to the image nearest the centre where the box leaves a periodic
-    // domain; a box over half the domain's length has no single nearest image
+    // Candidates are folded to the image nearest the centre where a target's sphere may leave the box,
+    // the condition of the exact predicate; a search box over half the domain's length has no single
+    // nearest image.  Folding rounds at 2^-53 of the domain's length: below 2^-24 of it, that is no
+    // longer small beside the rounding that `undecided` covers.
     GroupSearch  b{};
     const double S    = fmax(fmax(gh[0], gh[1]), gh[2]);
     bool         fold = false;
     exact             = exact || !(S > 0x1p-100 && S < 0x1p100);
     for (int d = 0; d < 3; ++d)
     {
-        if (!box.pbc[d]) continue;
         fold  = fold || gc[d] - gh[d] < box.lo[d] || gc[d] + gh[d] > box.hi[d];
-        exact = exact || gh[d] >= 0.4999 * box.len[d];
+        exact = exact || (box.pbc[d] && gh[d] >= 0.4999 * box.len[d]);
     }
+    fold = fold && box.anyPbc;
+    for (int d = 0; d < 3; ++d)
+        exact = exact || (fold && box.pbc[d] && S < 0x1p-24 * box.len[d]);
     b.cx = gc[0], b.cy = gc[1], b.cz = gc[2], b.inv = 1.0 / S;
     // 2^-20 covers the rounding of the half-widths, 2^-17 that of the distances
     b.hwx = fmaxf(float((gh[0] - rmin) * b.inv), 0.f) + 0x1p-20f;
@@ -753,9 +757,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6))) void ns
 // reference predicate d^2 < (2h)^2 is evaluated in FP64 with separately rounded operations
 // (findneighbors.hpp:33-60,115-140), so the neighbor sets are bit-identical to the CPU path.
 //
-// Groups without a single nearest periodic image, without a usable search box, or with a
-// target beyond ngmax neighbors (whose lists keep the first ngmax) are left to
-// nsCandidatesExact by overList.
+// Groups without a single nearest periodic image, with a candidate outside a periodic domain, without
+// a usable search box, or with a target beyond ngmax neighbors (whose lists keep the first ngmax) are
+// left to nsCandidatesExact by overList.
 //
 // One wave per group with the predicate in FP64 for all pairs (nsCandidatesExact) took 4.66 ms at
 // 256^3 and 0.185 ms for 4,096 particles, where it leaves most of the chip idle; this takes 3.50
@@ -972,6 +976,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void n
         }
     };
     loadChunks(0u);
+    uint64_t leave = 0;               // nonzero: the group is left to nsCandidatesExact
     uint32_t avail = 0, proc = 0;     // entries put into the ring, entries tested
     uint32_t ringIn = 0, ringOut = 0; // avail and proc modulo the ring's size
     for (uint32_t fill = 0;; fill += NS_CHUNKS)
@@ -986,6 +991,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void n
             double dx = ax[c] - sb.cx, dy = ay[c] - sb.cy, dz = az[c] - sb.cz;
             if (sb.fold)
             {
+                // a candidate outside the domain: the predicate folds it for some targets only
+                bool away = false;
+                if (box.pbc[0]) away = away | (ax[c] < box.lo[0]) | (ax[c] > box.hi[0]);
+                if (box.pbc[1]) away = away | (ay[c] < box.lo[1]) | (ay[c] > box.hi[1]);
+                if (box.pbc[2]) away = away | (az[c] < box.lo[2]) | (az[c] > box.hi[2]);
+                leave |= ballot(away & (lane < len[c]));
                 dx -= px * rint(dx * box.ilen[0]);
                 dy -= py * rint(dy * box.ilen[1]);
                 dz -= pz * rint(dz * box.ilen[2]);
@@ -1124,10 +1135,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void n
 
     count += uint32_t(__shfl_xor(int(count), 16, 64));
     count += uint32_t(__shfl_xor(int(count), 32, 64));
-    if constexpr (Sph)
+    if constexpr (Sph) leave |= ballot(count > ngmax || queued + 64u > out.capU);
+    if (Sph || sb.fold)
     {
-        const uint64_t over = ballot(count > ngmax || queued + 64u > out.capU);
-        if (lane == 0) wflag[q] = over != 0;
+        if (lane == 0) wflag[q] = leave != 0;
         __syncthreads();
         if (wflag[0] | wflag[1] | wflag[2] | wflag[3])
         {
@@ -1138,6 +1149,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void n
             }
             return;
         }
+    }
+    if constexpr (Sph)
+    {
         if (lane == 0) out.usize[sg] = queued;
         bool redo = false;
         if (act && part == 0)

@@ -210,3 +210,38 @@ def test_particles_with_nan_positions_are_no_neighbors(ctx, entry, periodic):
     nb, nc, ref, ref_nc = search_both(ctx, x, y, z, h, box, keys, entry, 400)
     assert not ref_nc[bad].any()
     assert_same_lists(np.ones(3000, bool), nb, nc, ref, ref_nc)
+
+
+@pytest.mark.parametrize("entry", ["plain", "fp64", "mixed"])
+@pytest.mark.parametrize("kind", ["outside", "tiny"])
+def test_folded_candidates(ctx, entry, kind):
+    """Targets at the faces of a periodic box.  outside: some particles lie up to a third of h outside of it;
+    the predicate folds offsets for the targets whose sphere leaves the box, and for those only.  tiny: all
+    particles within 1e-13 of a face, where folding rounds at 1e-3 of their distances."""
+    print("case fold", entry, kind, flush=True)
+    rng, n = np.random.default_rng(7), 3000
+    p = rng.random((n, 3))
+    h = np.full(n, 0.5 * (40 / (4 / 3 * np.pi * n)) ** (1 / 3))
+    if kind == "outside":
+        for i in np.flatnonzero(rng.random(n) < 0.05):
+            p[i, rng.integers(0, 3)] = 1.0 + 0.02 * rng.random() if rng.random() < 0.5 else -0.02 * rng.random()
+    else:
+        p[:, 0] -= 0.5
+        p *= 1e-13
+        p[:, 0] += np.where(p[:, 0] < 0, 1.0, 0.0)
+        h *= 1e-13
+    if entry == "mixed":
+        h = h.astype(np.float32).astype(np.float64)
+    box = oracle.Box.cube(0.0, 1.0, oracle.BC_PERIODIC)
+    keys, order = CPU.sort_by_key(CPU.sfc_keys(*(np.ascontiguousarray(p[:, d]) for d in range(3)), box),
+                                  np.arange(n, dtype=np.uint32))
+    x, y, z = (np.ascontiguousarray(p[order, d]) for d in range(3))
+    h = np.ascontiguousarray(h[order])
+    nb, nc, _, _ = search_both(ctx, x, y, z, h, box, keys, entry, 400)
+    for i in range(n):
+        d = [a - a[i] for a in (x, y, z)]
+        if not all(a[i] - 2.0 * h[i] >= 0.0 and a[i] + 2.0 * h[i] <= 1.0 for a in (x, y, z)):
+            d = [a - np.rint(a) for a in d]
+        hit = d[0] * d[0] + d[1] * d[1] + d[2] * d[2] < 4.0 * h[i] * h[i]
+        hit[i] = False
+        assert np.array_equal(nb[i, :nc[i]], np.flatnonzero(hit)), i
