@@ -12,8 +12,10 @@
 //                   rounded operations (findneighbors.hpp:33-60,115-140), so the neighbor sets are bit-identical to the CPU path; hits are
 //                   appended in ascending j, which is also the CPU's depth-first
 //                   order, so truncation at ngmax keeps the same entries.
-//   nsCandidatesExact : the same result with FP64 tests only, for groups whose search box
-//                   has no single nearest image, extreme units, or too many pieces.
+//   nsCandidatesExact : the same result with FP64 tests only, for groups with a list to be cut at
+//                   ngmax (targets that stay beyond it after the h iteration), whose search box
+//                   has no single nearest image, with candidates outside a periodic domain, with
+//                   extreme units, or with too many pieces.
 // The smoothing-length iteration of findNeighborsSph (sph/find_neighbors.hpp:10-41)
 // re-runs only the groups that still have particles outside [ng0/4, ngmax + 1].
 #include <algorithm>
@@ -759,7 +761,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6))) void ns
 //
 // Groups without a single nearest periodic image, with a candidate outside a periodic domain, without
 // a usable search box, or with a target beyond ngmax neighbors (whose lists keep the first ngmax) are
-// left to nsCandidatesExact by overList.
+// left to nsCandidatesExact by overList; the last not while a target of the group is still to be
+// searched again, where only the counts matter (1 M particles, h for 300 neighbors at first, ngmax 150:
+// 7.2 ms with the exact kernel in each of the iterations, now 2.7).
 //
 // One wave per group with the predicate in FP64 for all pairs (nsCandidatesExact) took 4.66 ms at
 // 256^3 and 0.185 ms for 4,096 particles, where it leaves most of the chip idle; this takes 3.50
@@ -1135,12 +1139,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void n
 
     count += uint32_t(__shfl_xor(int(count), 16, 64));
     count += uint32_t(__shfl_xor(int(count), 32, 64));
-    if constexpr (Sph) leave |= ballot(count > ngmax || queued + 64u > out.capU);
+    // A target beyond ngmax neighbors, whose list keeps the first ngmax, needs the exact kernel.  Where a
+    // target of the group is going to be searched again with another h, the whole group is, and the
+    // counts are all that this pass is for.
+    bool redo = false;
+    if constexpr (Sph)
+    {
+        if (act && part == 0)
+        {
+            const uint32_t ncSph = count + 1, ngmin = ng0 / 4;
+            redo = ((ngmin > ncSph) || (ncSph - 1 > ngmax)) && iter[i] < 10;
+        }
+    }
+    uint32_t state = 0; // 1: searched again, 2: a list too long, 4: not decided by the FP32 tests
     if (Sph || sb.fold)
     {
-        if (lane == 0) wflag[q] = leave != 0;
+        uint32_t mine = leave ? 4u : 0u;
+        if constexpr (Sph) mine |= (ballot(redo) ? 1u : 0u) | (ballot(count > ngmax || queued + 64u > out.capU) ? 2u : 0u);
+        if (lane == 0) wflag[q] = mine;
         __syncthreads();
-        if (wflag[0] | wflag[1] | wflag[2] | wflag[3])
+        state = wflag[0] | wflag[1] | wflag[2] | wflag[3];
+        if (state == 2u || (state & 4u))
         {
             if (threadIdx.x == 0)
             {
@@ -1153,32 +1172,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void n
     if constexpr (Sph)
     {
         if (lane == 0) out.usize[sg] = queued;
-        bool redo = false;
-        if (act && part == 0)
+        if (act && part == 0) nc[i] = count + 1; // dataset counts are indexed by particle (sph/find_neighbors.hpp:51)
+        if (redo)
         {
-            uint32_t ncSph = count + 1;
-            uint32_t ngmin = ng0 / 4;
-            bool     outR  = (ngmin > ncSph) || (ncSph - 1 > ngmax);
-            nc[i] = ncSph; // dataset counts are indexed by particle (sph/find_neighbors.hpp:51)
-            if (outR && iter[i] < 10)
+            // updateH (sph/kernels.hpp:27-33) in the precision of h, factor from the table
+            Th hn = h[i];
+            if (updateHTab(hfac, count + 1, hn))
             {
-                // updateH (sph/kernels.hpp:27-33) in the precision of h, factor from the table
-                Th hn = h[i];
-                if (updateHTab(hfac, ncSph, hn))
-                {
-                    h[i] = hn;
-                    iter[i] += 1;
-                    redo = true;
-                }
-                else
-                    flags->hfacMiss = 1;
+                h[i] = hn;
+                iter[i] += 1;
             }
+            else
+                flags->hfacMiss = 1;
         }
-        const uint64_t anyRedo = ballot(redo);
-        __syncthreads(); // wflag is read
-        if (lane == 0) wflag[q] = anyRedo != 0;
-        __syncthreads();
-        if (threadIdx.x == 0 && (wflag[0] | wflag[1] | wflag[2] | wflag[3])) redoList[atomicAdd(&flags->redoCount, 1u)] = g;
+        if (threadIdx.x == 0 && (state & 1u)) redoList[atomicAdd(&flags->redoCount, 1u)] = g;
     }
     else
     {

@@ -245,3 +245,37 @@ def test_folded_candidates(ctx, entry, kind):
         hit = d[0] * d[0] + d[1] * d[1] + d[2] * d[2] < 4.0 * h[i] * h[i]
         hit[i] = False
         assert np.array_equal(nb[i, :nc[i]], np.flatnonzero(hit)), i
+
+
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+def test_groups_searched_again_need_counts_only(ctx, prec):
+    """Initial h of five times as many neighbors as ngmax takes: every target's count exceeds it for some
+    iterations, and h follows the oracle; none of those lists is searched by the slower exact kernel."""
+    from sphexa_amd import hydro
+    from sphexa_amd._lib import FP64, MIXED
+
+    print("case h iteration", prec, flush=True)
+    n, ng0, ngmax = 20000, 60, 100
+    x, y, z, h, box, keys = sorted_cloud(n, prec, ng=500, periodic=False)
+    gbox = hydro.make_box([box.xmin, box.ymin, box.zmin], [box.xmax, box.ymax, box.zmax], [box.bx, box.by, box.bz])
+    t = hydro.tree_from_keys(ctx, torch.from_numpy(keys.view(np.int64)).to("cuda"), gbox, 64)
+    d = hydro.ParticlesData(n, MIXED if prec == "mixed" else FP64, ng0=ng0, ngmax=ngmax)
+    d.x, d.y, d.z, d.h = dev(x), dev(y), dev(z), dev(h, d.dtype)
+    d.allocate("cuda")
+    ctx.set_timing(True)
+    try:
+        ctx.timing_summary()
+        hydro.find_neighbors_sfc(ctx, d, gbox, t)
+        launches = {k: v[0] for k, v in ctx.timing_summary().items()}
+    finally:
+        ctx.set_timing(False)
+    rt = CPU.tree(keys, box)
+    nb, nc = u32(hydro.export_neighbors(ctx, d)), u32(d.nc)
+    if prec == "fp64":
+        _, ref_nc, ref_h = CPU.find_neighbors_sph(x, y, z, h, box, rt, ng0, ngmax)
+        assert np.array_equal(d.h.cpu().numpy(), ref_h) and np.array_equal(nc, ref_nc)
+    assert (nc <= ngmax + 1).all() and launches["nsCandidates"] > 2
+    final, _ = CPU.find_neighbors(x, y, z, d.h.double().cpu().numpy(), box, rt, ngmax)
+    bad = [i for i in range(n) if not np.array_equal(nb[i, :nc[i] - 1], final[i, :nc[i] - 1])]
+    assert not bad, bad[:10]
+    assert launches.get("nsCandidatesExact", 0) == 0
