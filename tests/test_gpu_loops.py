@@ -159,3 +159,38 @@ def test_ve_pairs(length, clean):
         for f in ref:
             scale = max(ref[k].abs().max() for k in GROUPS[0]) if f in GROUPS[0] else ref[f].abs().max()
             assert ((got[f] - ref[f]).abs() <= tol * scale).all(), (f, tol)
+
+
+@pytest.mark.parametrize("n,ng", [(4096, 100), (330_007, 800)])  # FP64: the table itself, the fitted table
+def test_coincident_particles_std(n, ng):
+    """Pairs at distance 0 (W(0), no direction, no approach speed) add nothing but to the sums of W: against the
+    FP64-exact loops.  FP64: the suite's 1e-10; mixed: the mode's 1e-3 (both of the largest value)."""
+    from sphexa_amd import hydro
+    from sphexa_amd._lib import FP64, MIXED
+
+    print("case coincident std", n, flush=True)
+    inp, b = uniform_box(n, seed=29, ng=ng)
+    for k in "xyz":
+        inp[k][1:400:2] = inp[k][0:400:2]
+    inp = {k: v if k in "xyz" else v.astype(np.float32).astype(np.float64) for k, v in inp.items()}
+    box = hydro.make_box([b.xmin, b.ymin, b.zmin], [b.xmax, b.ymax, b.zmax], [b.bx, b.by, b.bz])
+    out = []
+    for prec, exact in ((FP64, False), (MIXED, False), (FP64, True)):
+        ctx = hydro.Context(0)
+        try:
+            ctx.set_fp64_exact(exact)
+            step = hydro.HydroStep(ctx, n, box, prec, ng0=ng, ngmax=ng + ng // 2)
+            d_inp = {k: torch.from_numpy(np.ascontiguousarray(v)).to("cuda", torch.float64 if k in "xyz" else step.d.dtype)
+                     for k, v in inp.items()}
+            step.compute_forces(d_inp)
+            assert (ctx.candidate_tests() >= 5e8) == (ng == 800)
+            out.append({f: field(step, f) for f in STD})
+            out[-1]["minDt"] = torch.tensor(step.d.minDtCourant, dtype=torch.float64)
+        finally:
+            ctx.close()
+    ref = out.pop()
+    for got, tol in zip(out, (1e-10, 1e-3)):
+        for f in ref:
+            assert torch.isfinite(got[f]).all(), (f, tol)
+            group = next((g for g in GROUPS if f in g), (f,))
+            assert ((got[f] - ref[f]).abs() <= tol * max(ref[g].abs().max() for g in group)).all(), (f, tol)
