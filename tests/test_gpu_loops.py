@@ -194,3 +194,40 @@ def test_coincident_particles_std(n, ng):
             assert torch.isfinite(got[f]).all(), (f, tol)
             group = next((g for g in GROUPS if f in g), (f,))
             assert ((got[f] - ref[f]).abs() <= tol * max(ref[g].abs().max() for g in group)).all(), (f, tol)
+
+
+# particle mass, box length, specific energy: p / (kx m^2) and 1/h^3 are within the FP32 range, their product is not
+@pytest.mark.parametrize("mass,length,u", [(1e-9, 1e-4, 0.4), (1e15, 1e6, 1.0), (1.0 / 4096, 1.0, 1.0)])
+@pytest.mark.parametrize("clean", [False, True])
+def test_mixed_ve_units(mass, length, u, clean):
+    """Mixed VE accelerations and energy rates in systems of units with small and large particle masses, against
+    the FP64 loops; tolerance of the mode, 2e-3 of the largest value, as test_ve_pairs."""
+    from sphexa_amd import hydro
+    from sphexa_amd._lib import FP64, MIXED
+
+    print("case ve units", mass, length, clean, flush=True)
+    n = 4096
+    inp, b = uniform_box(n, seed=31, ng=100, hi=length)
+    inp["m"] = np.full(n, mass)
+    inp["u"] = np.full(n, u)
+    for k in ("vx", "vy", "vz"):
+        inp[k] = inp[k] * np.sqrt(u)
+    inp["alpha"] = np.random.default_rng(31).uniform(0.05, 1.0, n)
+    inp = {k: v if k in "xyz" else v.astype(np.float32).astype(np.float64) for k, v in inp.items()}
+    box = hydro.make_box([b.xmin, b.ymin, b.zmin], [b.xmax, b.ymax, b.zmax], [b.bx, b.by, b.bz])
+    out = []
+    for prec in (MIXED, FP64):
+        ctx = hydro.Context(0)
+        try:
+            step = hydro.VeHydroStep(ctx, n, box, prec, grad_v=True, av_clean=clean, ng0=100)
+            d_inp = {k: torch.from_numpy(np.ascontiguousarray(v)).to("cuda", torch.float64 if k in "xyz" else step.d.dtype)
+                     for k, v in inp.items()}
+            step.compute_forces(d_inp, dt=1e-4 * length)
+            out.append({f: field(step, f) for f in ("prho", "ax", "ay", "az", "du")})
+        finally:
+            ctx.close()
+    got, ref = out
+    assert torch.isfinite(got["prho"]).all() and (got["prho"] != 0).all()  # the field itself is in range
+    for f in ("ax", "ay", "az", "du"):
+        scale = max(ref[k].abs().max() for k in GROUPS[0]) if f in GROUPS[0] else ref[f].abs().max()
+        assert ((got[f] - ref[f]).abs() <= 2e-3 * scale).all(), f
