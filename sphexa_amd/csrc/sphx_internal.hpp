@@ -178,6 +178,7 @@ struct sphx_ctx
     sphx::SphLists  nsLists;
     uint32_t        nsNgmax = 0;
     const uint32_t* nsNc    = nullptr;
+    double          nsListTests = 0; // candidate tests of the passes that made nsLists, which grow with their pairs
     bool            nsValid = false;
     int             fp64Exact = 0; // 1: FP64 loops without FMA contraction (bit-exact vs the CPU path)
     int             loopShape[2] = {0, 0}; // per precision (FP64, MIXED): 0 LDS-staged, 1 sequential

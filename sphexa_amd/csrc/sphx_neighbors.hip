@@ -43,6 +43,7 @@ struct NsFlags
     uint32_t           retryCount; // groups that exceeded the small traversal capacities
     uint32_t           hfacMiss;   // a count to update h from lies beyond the factor table
     unsigned long long tests;      // (target, candidate) distance tests of this pass
+    unsigned long long listTests;  // after the first pass: those of every group's last pass
     uint32_t           overCount;  // groups that nsCandidates leaves to nsCandidatesExact
 };
 
@@ -694,9 +695,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6))) void ns
         if (done) break;
     }
     // exact pair tests of this pass
-    // (stored per launched group and summed by nsSumTests: one atomic per group on a
-    // single counter would serialize)
-    if (lane == 0) groupTests[blk] = tests;
+    // (stored per group and summed by nsSumTests: one atomic per group on a single counter
+    // would serialize)
+    if (lane == 0) groupTests[g] = tests;
 
     if constexpr (Sph)
     {
@@ -835,7 +836,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void n
         if (threadIdx.x == 0)
         {
             overList[atomicAdd(&flags->overCount, 1u)] = g;
-            groupTests[blk]                            = 0;
+            groupTests[g]                              = 0;
         }
         return;
     }
@@ -1133,9 +1134,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void n
         waveFence();
         masks(nb);
     }
-    // pair tests of this pass (stored per launched group and summed by nsSumTests: one atomic
-    // per group on a single counter would serialize)
-    if (threadIdx.x == 0) groupTests[blk] = (unsigned long long)avail * (e - s);
+    // pair tests of this pass (stored per group and summed by nsSumTests: one atomic per group on
+    // a single counter would serialize)
+    if (threadIdx.x == 0) groupTests[g] = (unsigned long long)avail * (e - s);
 
     count += uint32_t(__shfl_xor(int(count), 16, 64));
     count += uint32_t(__shfl_xor(int(count), 32, 64));
@@ -1164,7 +1165,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void n
             if (threadIdx.x == 0)
             {
                 overList[atomicAdd(&flags->overCount, 1u)] = g;
-                groupTests[blk]                            = 0;
+                groupTests[g]                              = 0;
             }
             return;
         }
@@ -1208,6 +1209,7 @@ __global__ void nsResetFlags(NsFlags* f, int clearErrors)
         f->retryCount = 0;
         f->overCount  = 0;
         f->tests      = 0;
+        f->listTests  = 0;
         if (clearErrors)
         {
             f->overflow = 0;
@@ -1217,21 +1219,22 @@ __global__ void nsResetFlags(NsFlags* f, int clearErrors)
     }
 }
 
-// flags->tests += sum of the per-group test counts (one atomic per block)
-__global__ __launch_bounds__(256) void nsSumTests(const unsigned long long* __restrict__ groupTests, uint32_t n,
-                                                  NsFlags* __restrict__ f)
+// *sum += the test counts of the n groups of list (nullptr: the first n), one atomic per block
+__global__ __launch_bounds__(256) void nsSumTests(const unsigned long long* __restrict__ groupTests,
+                                                  const uint32_t* __restrict__ list, uint32_t n,
+                                                  unsigned long long* __restrict__ sum)
 {
     __shared__ unsigned long long part[4];
     unsigned long long            v = 0;
     for (uint32_t k = blockIdx.x * 256u + threadIdx.x; k < n; k += gridDim.x * 256u)
-        v += groupTests[k];
+        v += groupTests[list ? list[k] : k];
     v = waveSum(v);
     if ((threadIdx.x & 63u) == 0) part[threadIdx.x >> 6] = v;
     __syncthreads();
     if (threadIdx.x == 0)
     {
         unsigned long long tot = part[0] + part[1] + part[2] + part[3];
-        if (tot) atomicAdd(&f->tests, tot);
+        if (tot) atomicAdd(sum, tot);
     }
 }
 
@@ -1355,9 +1358,10 @@ __global__ __launch_bounds__(256) void grpBoundaries(uint32_t first, uint32_t la
 
 // ---------------------------------------------------------------------------
 // host driver shared by both entry points
-static int sumTests(sphx_ctx* ctx, const unsigned long long* gtests, uint32_t n, NsFlags* flags)
+static int sumTests(sphx_ctx* ctx, const unsigned long long* gtests, const uint32_t* list, uint32_t n,
+                    unsigned long long* sum)
 {
-    nsSumTests<<<std::min<uint32_t>(256u, (n + 1023u) / 1024u), 256, 0, ctx->stream>>>(gtests, n, flags);
+    nsSumTests<<<std::min<uint32_t>(256u, (n + 1023u) / 1024u), 256, 0, ctx->stream>>>(gtests, list, n, sum);
     SPHX_LAUNCH_CHECK(ctx, "nsSumTests");
     return SPHX_OK;
 }
@@ -1365,8 +1369,10 @@ static int sumTests(sphx_ctx* ctx, const unsigned long long* gtests, uint32_t n,
 template<class Th, bool Sph>
 static int runSearch(sphx_ctx* ctx, const GroupsDev& G, const double* x, const double* y, const double* z, Th* h,
                      const sphx_box* box, const sphx_octree* t, uint32_t ngmax, uint32_t ng0, uint32_t* nbrs,
-                     SphLists lists, uint32_t* nc)
+                     SphLists lists, uint32_t* nc, double* listTests)
 {
+    ctx->nsTests = 0;
+    *listTests   = 0;
     if (G.numGroups == 0) return SPHX_OK;
     uint32_t  numG   = G.numGroups;
     uint2*    ranges = scratchT<uint2>(ctx, S_NS_RANGES, size_t(numG) * NS_LCAP);
@@ -1391,7 +1397,6 @@ static int runSearch(sphx_ctx* ctx, const GroupsDev& G, const double* x, const d
     }
     nsResetFlags<<<1, 64, 0, ctx->stream>>>(flags, 1);
     SPHX_LAUNCH_CHECK(ctx, "nsResetFlags");
-    ctx->nsTests = 0;
 
     const uint32_t* list      = nullptr; // nullptr: all groups
     uint32_t        numLaunch = numG;
@@ -1421,7 +1426,9 @@ static int runSearch(sphx_ctx* ctx, const GroupsDev& G, const double* x, const d
                                                                       flags, gtests);
         }
         SPHX_LAUNCH_CHECK(ctx, "nsCandidates");
-        SPHX_TRY(sumTests(ctx, gtests, numLaunch, flags));
+        // the tests of this pass, and those behind the lists as they are now: every group's last pass
+        SPHX_TRY(sumTests(ctx, gtests, list, numLaunch, &flags->tests));
+        if (pass) SPHX_TRY(sumTests(ctx, gtests, nullptr, numG, &flags->listTests));
         NsFlags hf;
         SPHX_TRY(readBack(ctx, flags, &hf, sizeof(NsFlags)));
         if (hf.overCount && !hf.overflow && !hf.badGroup)
@@ -1433,10 +1440,13 @@ static int runSearch(sphx_ctx* ctx, const GroupsDev& G, const double* x, const d
                                                                                  outList, flags, gtests);
             }
             SPHX_LAUNCH_CHECK(ctx, "nsCandidatesExact");
-            SPHX_TRY(sumTests(ctx, gtests, hf.overCount, flags));
+            // (nsCandidates left 0 for these groups)
+            SPHX_TRY(sumTests(ctx, gtests, over, hf.overCount, &flags->tests));
+            if (pass) SPHX_TRY(sumTests(ctx, gtests, over, hf.overCount, &flags->listTests));
             SPHX_TRY(readBack(ctx, flags, &hf, sizeof(NsFlags)));
         }
         ctx->nsTests += double(hf.tests);
+        *listTests = double(pass ? hf.listTests : hf.tests);
         if (hf.overflow) return fail(ctx, SPHX_ERR_STACK, "neighbor search: traversal capacity exceeded");
         if (hf.badGroup) return argError(ctx, "neighbor search: a target group holds more than 64 particles");
         if (hf.hfacMiss)
@@ -1547,8 +1557,9 @@ int sphx_find_neighbors(sphx_ctx* ctx, const double* x, const double* y, const d
     if (!validTree(tree)) return argError(ctx, "find_neighbors: incomplete tree view");
     GroupsDev G;
     SPHX_TRY(groupsFromArgs(ctx, nullptr, first, last, G));
+    double listTests; // (of no interest: the lists go to the caller)
     return runSearch<double, false>(ctx, G, x, y, z, const_cast<double*>(h), box, tree, ngmax, 0, nbrs, SphLists{},
-                                    nc);
+                                    nc, &listTests);
 }
 
 int sphx_find_neighbors_sph(sphx_ctx* ctx, const sphx_groups* groups, sphx_particles* d, const sphx_box* box,
@@ -1573,13 +1584,14 @@ int sphx_find_neighbors_sph(sphx_ctx* ctx, const sphx_groups* groups, sphx_parti
     L.unions = scratchT<uint32_t>(ctx, S_NS_UNION, numSub * L.capU);
     L.usize  = scratchT<uint32_t>(ctx, S_NS_USIZE, numSub);
     if (!L.masks || !L.unions || !L.usize) return SPHX_ERR_NOMEM;
-    int st;
+    int    st;
+    double listTests;
     if (d->precision == SPHX_FP64)
         st = runSearch<double, true>(ctx, G, d->x, d->y, d->z, static_cast<double*>(d->h), box, tree, d->ngmax,
-                                     d->ng0, nullptr, L, d->nc);
+                                     d->ng0, nullptr, L, d->nc, &listTests);
     else if (d->precision == SPHX_MIXED)
         st = runSearch<float, true>(ctx, G, d->x, d->y, d->z, static_cast<float*>(d->h), box, tree, d->ngmax,
-                                    d->ng0, nullptr, L, d->nc);
+                                    d->ng0, nullptr, L, d->nc, &listTests);
     else
         return argError(ctx, "find_neighbors_sph: unknown precision");
     if (st != SPHX_OK) return st;
@@ -1587,6 +1599,7 @@ int sphx_find_neighbors_sph(sphx_ctx* ctx, const sphx_groups* groups, sphx_parti
     ctx->nsValid  = true;
     ctx->nsGroups = G;
     ctx->nsNgmax  = d->ngmax;
+    ctx->nsListTests = listTests;
     ctx->nsNc     = d->nc;
     return SPHX_OK;
 }

@@ -231,3 +231,51 @@ def test_mixed_ve_units(mass, length, u, clean):
     for f in ("ax", "ay", "az", "du"):
         scale = max(ref[k].abs().max() for k in GROUPS[0]) if f in GROUPS[0] else ref[f].abs().max()
         assert ((got[f] - ref[f]).abs() <= 2e-3 * scale).all(), f
+
+
+def test_loop_form_follows_the_lists():
+    """The FP64 loops' form (the table, or its fit) depends on the lists that they run on, not on what else the
+    context searched: a plain search in between, and one of no targets, leave every bit as it is; a second set's
+    short lists take the table, also where h iterated to them over longer ones."""
+    from sphexa_amd import hydro
+    from sphexa_amd._lib import FP64
+
+    def lists_of(ctx, n, ng, start=1.0):
+        inp, b = uniform_box(n, seed=37, ng=ng)
+        t = {k: torch.from_numpy(v).to("cuda") for k, v in inp.items()}
+        keys = hydro.compute_sfc_keys(ctx, t["x"], t["y"], t["z"], box)
+        order = hydro.sequence(ctx, n)
+        hydro.sort_by_key(ctx, keys, order)
+        d = hydro.ParticlesData(n, FP64, ng0=ng, ngmax=ng + ng // 2)
+        for f in ("x", "y", "z", "h", "m"):
+            setattr(d, f, hydro.gather(ctx, order, t[f]))
+        d.h *= start ** (1 / 3)
+        d.allocate("cuda")
+        tree = hydro.tree_from_keys(ctx, keys, box, 64)
+        hydro.find_neighbors_sfc(ctx, d, box, tree)
+        return d, tree
+
+    print("case loop form", flush=True)
+    ctx = hydro.Context(0)
+    try:
+        box = hydro.make_box(0.0, 1.0, 1)
+        d, tree = lists_of(ctx, 330_007, 800)
+        ctx.set_timing(True)
+
+        def density():
+            ctx.timing_summary()
+            hydro.compute_density(ctx, d, box)
+            return d.rho.clone(), "tableFitKernel" in ctx.timing_summary()
+
+        rho, fitted = density()
+        assert fitted
+        for last in (100, 0):
+            hydro.find_neighbors(ctx, d.x, d.y, d.z, d.h, box, tree, 16, 0, last)
+            again, fitted = density()
+            assert fitted and torch.equal(rho, again), last
+        d, _ = lists_of(ctx, 1000, 50)
+        assert not density()[1]
+        d, _ = lists_of(ctx, 100_000, 500, start=2.6)
+        assert ctx.candidate_tests() >= 5e8 and not density()[1]
+    finally:
+        ctx.close()
