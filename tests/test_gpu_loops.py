@@ -279,3 +279,50 @@ def test_loop_form_follows_the_lists():
         assert ctx.candidate_tests() >= 5e8 and not density()[1]
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("kind", ["std", "ve"])
+def test_fitted_table_at_the_rim(kind):
+    """Targets whose neighbors all lie at 1.985 to 1.995 h, where W is 1e-14 of W(0), beside a cloud whose long
+    lists take the fitted table: sums of such weights keep the relative accuracy that the table itself has (1e-10
+    of the largest value among these targets, as for the others in test_fitted_table_loops_equal_table_loops; a
+    distance rounds W by 6 * 2^-53 * 200 = 1e-13 there).  Not gradh, and a and du by it: 1 minus the own terms'
+    share, 5e-11, is what rounding leaves of it in either form."""
+    from sphexa_amd import hydro
+    from sphexa_amd._lib import FP64
+
+    print("case rim", kind, flush=True)
+    inp, b = uniform_box(330_007, seed=41, periodic=False, ng=800)
+    rng, side, h = np.random.default_rng(41), 8, 0.25 * inp["h"][0]
+    grid = np.stack(np.meshgrid(*[np.arange(side)] * 3, indexing="ij"), -1).reshape(-1, 3) * 1.99 * h
+    grid += rng.uniform(-0.001, 0.001, grid.shape) * h + [0.3, 0.3, 1.5]
+    k = len(grid)
+    more = dict(x=grid[:, 0], y=grid[:, 1], z=grid[:, 2], h=np.full(k, h), m=np.full(k, inp["m"][0]), u=np.ones(k),
+                **{v: rng.normal(0, 0.1, k) for v in ("vx", "vy", "vz")})
+    inp = {f: np.concatenate([inp[f], more[f]]) for f in inp}
+    n = len(inp["x"])
+    out = []
+    for shape in (0, 1):
+        ctx = hydro.Context(0)
+        try:
+            ctx.set_loop_shape(FP64, shape)
+            make = hydro.HydroStep if kind == "std" else hydro.VeHydroStep
+            step = make(ctx, n, hydro.make_box([0.0] * 3, [1.0, 1.0, 2.0], 0), FP64, ng0=16, ngmax=1200)
+            d_inp = {f: torch.from_numpy(np.ascontiguousarray(v)).to("cuda") for f, v in inp.items()}
+            if kind == "ve":
+                d_inp["alpha"] = torch.full_like(d_inp["x"], 0.3)
+            step.compute_forces(d_inp)
+            assert ctx.candidate_tests() >= 5e8
+            rim = step.d.z > 1.2
+            nc = step.d.nc[rim]
+            assert rim.sum() == k and nc.min() == 4 and nc.max() == 7
+            fields = STD if kind == "std" else [f for f in VE if f not in ("gradh", "ax", "ay", "az", "du")]
+            out.append({f: field(step, f)[rim] for f in fields})
+        finally:
+            ctx.close()
+    got, ref = out
+    for f in got:
+        group = next((g for g in GROUPS if f in g), (f,))
+        scale = max(ref[g].abs().max().item() for g in group)
+        err = (got[f] - ref[f]).abs().max().item() / scale
+        assert np.isfinite(scale) and err <= 1e-10, (f, err)
