@@ -339,21 +339,19 @@ int sphx_compute_hydro_std(sphx_ctx* ctx, const sphx_groups* groups, sphx_partic
     auto* dt = scratchT<unsigned long long>(ctx, S_SMALL, 4);
     if (!dt) return SPHX_ERR_NOMEM;
     // every particle a target: the density loop's epilogue writes the IAD records and, in
-    // mixed precision, the IAD loop's epilogue the momentum-energy records (the 144-byte
-    // FP64 records cost the FP64 IAD epilogue more than their packing launch: measured)
+    // mixed precision, the IAD loop's epilogue the momentum-energy records
     const bool handOff = G.first == 0 && G.last == d->n;
-    const bool meOff   = handOff && d->precision == SPHX_MIXED;
     const bool ex      = useExact(ctx, d);
     DBox       db      = makeDBox(box);
     SPHX_TRY(ex ? exact::launchDensity(ctx, G, lists, d, db, handOff)
                 : fast::launchDensity(ctx, G, lists, d, db, handOff));
     SPHX_TRY(launchEos(ctx, G.first, G.last, d));
-    SPHX_TRY(ex ? exact::launchIAD(ctx, G, lists, d, db, handOff, meOff)
-                : fast::launchIAD(ctx, G, lists, d, db, handOff, meOff));
+    SPHX_TRY(ex ? exact::launchIAD(ctx, G, lists, d, db, handOff, handOff)
+                : fast::launchIAD(ctx, G, lists, d, db, handOff, handOff));
     initMinDt<<<1, 64, 0, ctx->stream>>>(dt);
     SPHX_LAUNCH_CHECK(ctx, "initMinDt");
-    SPHX_TRY(ex ? exact::launchMomentumEnergy(ctx, G, lists, d, db, dt, meOff)
-                : fast::launchMomentumEnergy(ctx, G, lists, d, db, dt, meOff));
+    SPHX_TRY(ex ? exact::launchMomentumEnergy(ctx, G, lists, d, db, dt, handOff)
+                : fast::launchMomentumEnergy(ctx, G, lists, d, db, dt, handOff));
     return finishMinDt(ctx, dt, d);
 }
 
