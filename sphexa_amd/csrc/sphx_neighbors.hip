@@ -777,6 +777,7 @@ constexpr uint32_t NS_RING     = 64 + 64 * NS_CHUNKS; // 63 entries carried over
 // a wave's queue: two batches of 64 members (float4), 64 bytes of padding after each 16 of them
 // so that the masks' operand reads (members 16 apart) meet different banks
 constexpr uint32_t NS_QHALF = 64 * 4 + 4 * 16; // floats per batch
+static_assert(NS_QHALF % 4 == 0, "every wave's queue and both of its batches start at 16 bytes");
 
 using floatx4 = __attribute__((ext_vector_type(4))) float;
 
@@ -815,7 +816,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void n
 #pragma clang fp contract(off)
     __shared__ float4   ent[NS_RING];
     __shared__ uint32_t entJ[NS_RING];
-    __shared__ float    queAll[4][2 * NS_QHALF];
+    __shared__ alignas(16) float queAll[4][2 * NS_QHALF]; // (written 16 bytes at a time)
     __shared__ uint32_t queJAll[4][128];
     __shared__ uint32_t selfAll[4][16]; // the union index of each target
     __shared__ uint32_t wcnt[4], wflag[4];
