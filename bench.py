@@ -48,7 +48,7 @@ PEAK_FP32_TFLOPS = 157.3
 # algorithmic work per unit, counted from the reference pair loops
 # (mul/add/sub/div/sqrt = 1 flop, one table lookup = 7 flops)
 FLOP_PER_PAIR = {"densityKernel": 19.0, "iadKernel": 37.0, "momentumEnergyKernel": 121.0}
-FLOP_PER_TEST = 11.0  # neighbor candidate test, the reference's own convention
+FLOP_PER_DISTANCE = 11.0  # of a pair, once: what a search cannot do without (it tests more candidates)
 IAD_FLOP_PER_PARTICLE = 60.0
 
 
@@ -262,22 +262,21 @@ def roofline(kernels, pairs, n, steps, precision, tests):
     if name in FLOP_PER_PAIR:
         flop = FLOP_PER_PAIR[name] * pairs + (IAD_FLOP_PER_PARTICLE * n if name == "iadKernel" else 0.0)
         unit_note = f"{FLOP_PER_PAIR[name]:.0f} flop/pair x {pairs} pairs"
-    elif name == "nsCandidates" and tests:
-        flop = FLOP_PER_TEST * tests
-        unit_note = f"{FLOP_PER_TEST:.0f} flop/candidate test x {tests} tests"
+    elif name.startswith("nsCandidates") and tests:
+        # tests in FP32 on the matrix cores, in FP64 where that does not decide: a rate of tests, no flop rate
+        flop = None
+        unit_note = f"{tests:.0f} candidate tests, {tests / (per_launch_ms * 1e-3):.3g} per second"
     else:
         flop = None
         unit_note = "no algorithmic flop count"
-    # the neighbor predicate is FP64 in both precisions; the particle loops compute in
-    # the precision of the fields
-    fp64 = precision == 0 or name.startswith("ns")
-    peak = PEAK_FP64_TFLOPS if fp64 else PEAK_FP32_TFLOPS
+    # the particle loops compute in the precision of the fields
+    peak = (PEAK_FP64_TFLOPS if precision == 0 else PEAK_FP32_TFLOPS) if flop else None
     achieved = (flop / (per_launch_ms * 1e-3) / 1e12) if flop else None
     return {"kernel": name, "bound": "valu", "achieved": achieved, "peak": peak, "unit": "TFLOP/s",
             "frac": (achieved / peak) if achieved else None, "traffic": None, "per_launch_ms": per_launch_ms,
             "launches": launches, "work": unit_note,
-            "peak_note": "MI355X published vector peak for the kernel's arithmetic (FP64 78.6 for the "
-                         "neighbor search and the FP64 loops, FP32 157.3 for the mixed loops); MFMA runs only the search's distance tests"}
+            "peak_note": "MI355X published vector peak for the loops' arithmetic (78.6 FP64, 157.3 mixed); the "
+                         "neighbor search, whose distance tests run on MFMA, has a test rate only"}
 
 
 def measured_traffic(kernel, workload_tag):
@@ -523,15 +522,15 @@ def main():
         "kernels_ms_per_step": {k: round(v[1] / args.steps, 3) for k, v in R["kernels"].items()},
     }
     # whole-step algorithmic rates: pair flops of the three loops (19 + 37 + 121 per pair, 60 per
-    # particle for the IAD inverse), 11 flops per candidate test of the search, and the
+    # particle for the IAD inverse), 11 per pair for its distance in the search, and the
     # compulsory HBM bytes per particle of the step (keys, sort, permutation, loops)
     def step_totals(res, prec):
-        flop = (19.0 + 37.0 + 121.0) * res["pairs"] + IAD_FLOP_PER_PARTICLE * n + FLOP_PER_TEST * (res["tests"] or 0)
+        flop = (19.0 + 37.0 + 121.0) * res["pairs"] + IAD_FLOP_PER_PARTICLE * n + FLOP_PER_DISTANCE * res["pairs"]
         nbytes = (532.0 if prec == MIXED else 716.0) * n
         t = res["ms"] * 1e-3
         return {"algorithmic_TFLOPs": flop / t / 1e12, "compulsory_GBs": nbytes / t / 1e9,
                 "hbm_frac": nbytes / t / 1e9 / PEAK_HBM_GBS,
-                "note": "step flops = 177 per pair + 60 per particle + 11 per candidate test; compulsory bytes "
+                "note": "step flops = 188 per pair + 60 per particle; compulsory bytes "
                         f"{'532' if prec == MIXED else '716'} per particle"}
     out["step_totals"] = step_totals(R, main_prec)
     if FP64 in results and MIXED in results:
