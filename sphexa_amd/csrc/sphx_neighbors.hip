@@ -767,8 +767,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6))) void ns
 // 7.2 ms with the exact kernel in each of the iterations, now 2.7).
 //
 // One wave per group with the predicate in FP64 for all pairs (nsCandidatesExact) took 4.66 ms at
-// 256^3 and 0.185 ms for 4,096 particles, where it leaves most of the chip idle; this takes 3.50
-// and 0.025 ms.  Bound by instruction issue: 1,250 VALU and 700 SALU instructions per wave, 60 %
+// 256^3 and 0.185 ms for 4,096 particles, where it leaves most of the chip idle; this takes 3.51
+// and 0.027 ms.  Bound by instruction issue: 1,250 VALU and 700 SALU instructions per wave, 60 %
 // of the time with VALU work, the rest waits for the first chunks and the barriers of a step.
 // candidate chunks per wave and step: 2 (1: 3.6 ms at 256^3, more steps; 3: 4.1, registers)
 constexpr uint32_t NS_PER_WAVE = 2;
